@@ -326,8 +326,8 @@ int ltx_gemm_mx_gelu_mxfp8(const uint8_t* A, int64_t lda, const uint8_t* a_scale
                            const float* bias, uint8_t* Cq, int64_t ldcq, uint8_t* c_scale, int64_t ld_cscale,
                            int64_t M, int64_t N, int64_t K, int flags, void* stream);
 
-/* Split-K forms of the three GEMMs for few-row products (the 68-token audio
- * stream, 256-token contexts): `splits` blocks per 128x128 output tile each
+/* Split-K forms of the three GEMMs for products of few output tiles (the
+ * 68-token audio stream, short clips): `splits` blocks per output tile each
  * accumulate K / splits of the product into an fp32 partial tile in
  * `workspace` (ltx_gemm_splitk_workspace_bytes(M, N, splits) bytes, 16-byte
  * aligned, caller-owned), then one pass sums the partials in split order and
@@ -337,6 +337,9 @@ int ltx_gemm_mx_gelu_mxfp8(const uint8_t* A, int64_t lda, const uint8_t* a_scale
  * LTX_GEMM_TILE_128.  Same operand rules as above.
  */
 int64_t ltx_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int64_t splits);
+/* The split count the library would choose (1: one pass) for a product of
+ * weight format `wformat` (0 bf16, 1 int8, 2 MXFP8). */
+int ltx_gemm_auto_splits(int64_t M, int64_t N, int64_t K, int wformat);
 int ltx_gemm_splitk_bf16(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias,
                          void* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int epilogue,
                          const void* residual, int64_t ldr, const float* gate, int64_t sigmoid_from,

@@ -43,8 +43,6 @@
 //     round-robins workgroups over the 8 XCDs), grouped 4 tile-rows at a
 //     time: the 32 concurrent tiles of an XCD form 4 x 8, the fewest distinct
 //     activation and weight bytes per K step.
-#include <type_traits>
-
 #include "gemm_common.h"
 
 namespace ltx {
@@ -53,61 +51,7 @@ namespace ltx {
 // registers one stage ahead that are written to LDS during the next stage.
 enum Loader { LOAD_DMA = 0, LOAD_REG = 1 };
 
-struct GemmArgs {
-  const bf16* A;
-  int64_t lda;
-  const void* B;
-  int64_t ldb;
-  const void* bscale;  // int8: fp32 (N); mxfp8: uint8 (N, K/32)
-  int64_t ld_scale;    // mxfp8 scale row stride (bytes)
-  const float* bias;   // fp32 (N) or null
-  bf16* C;
-  int64_t ldc;
-  const bf16* R;       // residual (gated epilogues), may alias C
-  int64_t ldr;
-  const float* gate;   // fp32 (N)
-  int sig_from;        // columns n >= sig_from get the 2*sigmoid head-gate epilogue
-  int round_then_bias; // bias added to the bf16-rounded product (quantised-linear form)
-  float* partial;      // split-K: fp32 partial products [split][M][ldc], no epilogue
-  const uint8_t* ascale;  // B_MX: activation E8M0 scales (M, K/32)
-  int64_t ld_ascale;      // B_MX: their row stride (bytes)
-  uint8_t* cscale;        // kEpiGeluMx: output E8M0 scales (M, N/32); C holds the codes
-  int64_t ld_cscale;
-  int M, N, K;         // split-K: K is the per-split depth
-  int tiles_m, tiles_n;
-  // 8-wave bias epilogue: per-row sums of squares of the bf16 outputs of
-  // columns [0, ss_cols), one fp32 partial per 64-column slice at
-  // rowss[row * ld_rowss + col / 64] (null: none)
-  float* rowss = nullptr;
-  int64_t ld_rowss = 0;
-  int ss_cols = 0;
-};
-
 constexpr int kGemmThreads = 256;
-// EPI value of the split-K pass: the accumulators go to the fp32 partial
-// buffer as they are, the epilogue runs in splitk_epilogue_kernel.
-constexpr int kEpiPartial = 16;
-// EPI value of the MX kernel's FF up-projection: the GELU epilogue whose
-// bf16 result leaves as MXFP8 rows (codes in C, E8M0 scales in cscale) --
-// the next product's quantised activations, written by this one.
-constexpr int kEpiGeluMx = 5;
-constexpr int kGroupM = 4;
-
-__device__ __forceinline__ void tile_coords(int bid, int nblocks, int tiles_m, int tiles_n, int& tm,
-                                            int& tn) {
-  // XCD-contiguous renumbering: hardware sends block b to XCD b % 8.
-  const int q = nblocks / kNumXcd, r = nblocks % kNumXcd;
-  const int xcd = bid % kNumXcd, idx = bid / kNumXcd;
-  const int logical = xcd * q + (xcd < r ? xcd : r) + idx;
-  // grouped ordering: kGroupM tile-rows sweep the tile-columns together
-  const int per_group = kGroupM * tiles_n;
-  const int group = logical / per_group;
-  const int first_m = group * kGroupM;
-  const int gsize = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
-  const int in_group = logical % per_group;
-  tm = first_m + in_group % gsize;
-  tn = in_group / gsize;
-}
 
 template <int BM, int BN, int BK, int STAGES_, int BKIND, int EPI, int SWZ, int LOADER>
 struct GemmCfg {
@@ -756,32 +700,6 @@ constexpr int kG8Threads = 512;
 // the automatic tile choice uses the 8-wave kernel for 8-bit weights (MXFP8
 // and int8) on problems of at least 100 256x256 tiles, and for bf16 weights on
 // problems of at least 160
-
-// f(integral_constant<int, I>) for I = I0 .. N-1, in order
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
-
-// 16-byte chunk XOR of row r in the 8-wave kernel's stages, 64-byte rows (4
-// chunks) and 128-byte rows (8 chunks).  ds_read_b128 services a wave's lanes
-// 16 at a time, in the lane-octet pairs (0, 3), (1, 2), (4, 7), (5, 6)
-// (probed: two octets reading the same banks at other addresses conflict only
-// in those pairs), and its conflicts were probed per read pattern (rocprofv3
-// SQ_LDS_BANK_CONFLICT of a one-read kernel over 290 lane -> address tables):
-// the 32x32 fragment reads (lane = row 0-31, lane / 32 = chunk half) are
-// conflict-free under chunk ^ ((r / 4) % 4) and chunk ^ ((r / 2) % 8), but the
-// 16x16 reads (lane % 16 = row, lane / 16 = chunk quarter) conflict under
-// those (the FF up-projection: 36-39 M conflict cycles per launch) and not
-// under chunk ^ (r bit 0 | r bit 2 << 1) and chunk ^ (r bit 1 | r bit 0 << 1
-// | r bit 2 << 2).
-__device__ __forceinline__ int g8_swz64(int r, bool s16) { return s16 ? ((r & 1) | ((r >> 1) & 2)) : ((r >> 2) & 3); }
-__device__ __forceinline__ int g8_swz128(int r, bool s16) {
-  return s16 ? (((r >> 1) & 1) | ((r & 1) << 1) | (r & 4)) : ((r >> 1) & 7);
-}
 
 template <int BKIND, int BM_ = 256, int BF_STAGES = 5>
 struct G8Cfg {
@@ -1470,6 +1388,67 @@ static GemmArgs rows_from(const GemmArgs& p, int r0) {
   return q;
 }
 
+// ---- the mid-size kernel (gemm_kg.hip): which products, tile height, splits --
+// Operand extents within its 31-bit buffer record counts, whole units of 128 k
+// per split, and for MXFP8 whole groups of four units (16 E8M0 bytes) per
+// split in 4-byte aligned pieces.
+static bool kg_ok(int bkind, int64_t M, int64_t N, int64_t Ks, int64_t lda, int64_t ldb, int64_t ld_scale) {
+  const int64_t lim = (int64_t)1 << 31;
+  return bkind != B_MX && Ks > 0 && Ks % (bkind == B_MXFP8 ? 512 : 128) == 0 && M * lda * 2 < lim &&
+         N * ldb * (bkind == B_BF16 ? 2 : 1) < lim && (bkind != B_MXFP8 || N * ld_scale < lim);
+}
+
+// Modelled time (us) of a product on the mid-size kernel.  A round of one
+// workgroup per CU costs `unit` us per 128 k (measured alone at K = 4096,
+// tiles of 64 / 128 / 192 rows, one partial round), and however many rounds,
+// the L2s deliver about 13 TB/s of tile operands to the CUs (every shape with
+// all CUs busy measured 11-15 TB/s); 4 us of launch, first loads and
+// epilogue; split-K adds its second launch and one write and read of the fp32
+// partials.  Model against measured (MXFP8): 1296 x 4096 -> 4096 192 rows 40 /
+// 43, 128 rows 53 / 59, 64 rows 57 / 61; 1296 x 16384 -> 4096 148 / 150,
+// 201 / 193, 220 / 197; 204 x 8192 -> 2048 64 rows, 1 / 2 / 4 splits
+// 39 / 27 / 20 against 32 / 24 / 19.
+static double kg_time(int bkind, int64_t M, int64_t N, int64_t K, int bm, int64_t splits) {
+  static const double unit_us[3][3] = {{0.70, 0.88, 1.05}, {0.87, 1.00, 1.25}, {0.55, 0.77, 1.02}};
+  const int64_t wgs = ((M + bm - 1) / bm) * ((N + 127) / 128) * splits;
+  const double units = (double)(K / 128) / (double)splits;
+  const double rounds = (double)((wgs + 255) / 256);
+  const double bytes = (double)wgs * units * 128.0 * (bkind == B_BF16 ? 2.0 * (bm + 128) : 2.0 * bm + 128.0);
+  double t = rounds * units * unit_us[bkind][bm / 64 - 1];
+  if (bytes / 13e6 > t) t = bytes / 13e6;
+  t += 4.0;
+  if (splits > 1) t += 3.5 + (double)(M * N * splits) * 8.0 / 3.5e6;
+  return t;
+}
+
+// The tile height that the model finds fastest for a split count.
+static int kg_rows(int bkind, int64_t M, int64_t N, int64_t K, int64_t splits, double* us) {
+  int best = 64;
+  double t = kg_time(bkind, M, N, K, 64, splits);
+  for (int bm = 128; bm <= 192; bm += 64) {
+    const double u = kg_time(bkind, M, N, K, bm, splits);
+    if (u < t) {
+      t = u;
+      best = bm;
+    }
+  }
+  if (us) *us = t;
+  return best;
+}
+
+// Whether an automatic launch takes the mid-size kernel: below 160 tiles of
+// 256x256 (from there the 256-row tiles fill the chip; 3456 x 4096 -> 4096 90
+// against 121 us), except where the 8-wave kernel's single round of 100-159
+// tiles models faster (2.1 us per 128 k measured; int8 2.4).
+static bool kg_auto(int bkind, const GemmArgs& p) {
+  const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
+  if (big >= 160 || !kg_ok(bkind, p.M, p.N, p.K, p.lda, p.ldb, p.ld_scale)) return false;
+  if (big < 100) return true;
+  double us;
+  kg_rows(bkind, p.M, p.N, p.K, 1, &us);
+  return us < 4.0 + (p.K / 128) * (bkind == B_INT8 ? 2.4 : 2.1);
+}
+
 // Tile shapes (all K step 64): 256x256 and 128x128 with the register-staged
 // loader (1 and 2; 128x128 runs two workgroups per CU), 256x256 with the
 // LDS-DMA loader (3), 256x128 register-staged (4), and the 8-wave kernel with
@@ -1477,6 +1456,10 @@ static GemmArgs rows_from(const GemmArgs& p, int r0) {
 template <int BKIND, int EPI>
 static int launch_epi_w(const GemmArgs& p, int tile, hipStream_t s) {
   const bool auto_tile = tile == 0;
+  if (auto_tile && kg_auto(BKIND, p)) {
+    kg_launch(BKIND, p, EPI, kg_rows(BKIND, p.M, p.N, p.K, 1, nullptr), 1, s);
+    return LTX_OK;
+  }
   if (tile == 0) {
     // Large tiles when they still give most CUs a tile; 128x128 otherwise.
     // 8-bit weights take the 8-wave kernel from 100 tiles of 256x256: the A2V
@@ -1500,7 +1483,7 @@ static int launch_epi_w(const GemmArgs& p, int tile, hipStream_t s) {
     const bool g8 = (BKIND == B_MXFP8 || BKIND == B_INT8 || (BKIND == B_BF16 && (p.N >= p.K || big < 160))) &&
                     g8_ok<BKIND>(p);
     tile = big >= 160 ? (g8 ? 5 : 1) : (big >= 100 && g8 ? 5 : 2);
-    // row sums of squares come from the 8-wave kernel's epilogue only
+    // row sums of squares come from the 8-wave kernels' epilogues only
     if (p.rowss && tile != 5) tile = 5;
   }
   if (p.rowss && tile != 5 && tile != 6) return LTX_ERR_UNSUPPORTED;
@@ -1635,7 +1618,9 @@ template <int BKIND>
 static int launch_splitk(const GemmArgs& p0, int epilogue, int splits, float* workspace, hipStream_t s) {
   const int epi = epilogue & 0xff;
   const int tile = (epilogue >> 8) & 0xf;
-  if (tile != 0 && tile != 2) return LTX_ERR_UNSUPPORTED;  // 128x128 register-staged tiles
+  // the mid-size kernel, or (explicitly, and for what it does not take)
+  // 128x128 register-staged tiles
+  if (tile != 0 && tile != 2) return LTX_ERR_UNSUPPORTED;
   GemmArgs p = p0;
   p.round_then_bias = (epilogue & LTX_GEMM_ROUND_THEN_BIAS) != 0;
   // pass 1: partial products, per-split depth K / splits, row stride N
@@ -1645,8 +1630,11 @@ static int launch_splitk(const GemmArgs& p0, int epilogue, int splits, float* wo
   q.ldc = p.N;
   q.tiles_m = (p.M + 127) / 128;
   q.tiles_n = (p.N + 127) / 128;
-  gemm_kernel<128, 128, 64, 2, BKIND, kEpiPartial, 0, LOAD_REG>
-      <<<q.tiles_m * q.tiles_n * splits, kGemmThreads, 0, s>>>(q);
+  if (tile == 0 && kg_ok(BKIND, q.M, q.N, q.K, q.lda, q.ldb, q.ld_scale))
+    kg_launch(BKIND, q, kEpiPartial, kg_rows(BKIND, p.M, p.N, p.K, splits, nullptr), splits, s);
+  else
+    gemm_kernel<128, 128, 64, 2, BKIND, kEpiPartial, 0, LOAD_REG>
+        <<<q.tiles_m * q.tiles_n * splits, kGemmThreads, 0, s>>>(q);
   // pass 2: sum + epilogue
   p.partial = workspace;
   const int64_t vecs = (int64_t)p.M * (p.N / 8);
@@ -1863,6 +1851,32 @@ extern "C" int ltx_gemm_mx_gelu_mxfp8(const uint8_t* A, int64_t lda, const uint8
   p.cscale = c_scale;
   p.ld_cscale = ld_cscale;
   return launch_kind<B_MX>(p, kEpiGeluMx | flags, (hipStream_t)stream);
+}
+
+// Split-K factor that the library would choose for a product (wformat 0:
+// bf16, 1: int8, 2: MXFP8): the power of two that models fastest while the
+// splits still fit one round of the 256 CUs, taken over fewer splits only
+// when it models >= 15 % faster (a second launch and a workspace).
+extern "C" int ltx_gemm_auto_splits(int64_t M, int64_t N, int64_t K, int wformat) {
+  if (M <= 0 || N <= 0 || K <= 0 || wformat < 0 || wformat > 2 || M > INT32_MAX / 2 || N > INT32_MAX / 2 ||
+      K > INT32_MAX / 2)
+    return 1;
+  const int64_t ld_scale = wformat == B_MXFP8 ? K / 32 : 0;
+  if (((M + 255) / 256) * ((N + 255) / 256) >= 100 || !kg_ok(wformat, M, N, K, K, K, ld_scale)) return 1;
+  double best;
+  kg_rows(wformat, M, N, K, 1, &best);
+  int splits = 1;
+  for (int s = 2; s <= 16; s *= 2) {
+    if (K % s || !kg_ok(wformat, M, N, K / s, K, K, ld_scale)) break;
+    double us;
+    const int bm = kg_rows(wformat, M, N, K, s, &us);
+    if (((M + bm - 1) / bm) * ((N + 127) / 128) * s > 256) continue;
+    if (us < 0.85 * best) {
+      best = us;
+      splits = s;
+    }
+  }
+  return splits;
 }
 
 extern "C" int64_t ltx_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int64_t splits) {

@@ -3,6 +3,8 @@
 // arithmetic, E8M0 decoding, LDS-DMA / buffer-load helpers and wait counters.
 #pragma once
 
+#include <type_traits>
+
 #include "ltx_common.h"
 
 namespace ltx {
@@ -110,5 +112,90 @@ __device__ __forceinline__ void barrier_nofence() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+struct GemmArgs {
+  const bf16* A;
+  int64_t lda;
+  const void* B;
+  int64_t ldb;
+  const void* bscale;  // int8: fp32 (N); mxfp8: uint8 (N, K/32)
+  int64_t ld_scale;    // mxfp8 scale row stride (bytes)
+  const float* bias;   // fp32 (N) or null
+  bf16* C;
+  int64_t ldc;
+  const bf16* R;       // residual (gated epilogues), may alias C
+  int64_t ldr;
+  const float* gate;   // fp32 (N)
+  int sig_from;        // columns n >= sig_from get the 2*sigmoid head-gate epilogue
+  int round_then_bias; // bias added to the bf16-rounded product (quantised-linear form)
+  float* partial;      // split-K: fp32 partial products [split][M][ldc], no epilogue
+  const uint8_t* ascale;  // B_MX: activation E8M0 scales (M, K/32)
+  int64_t ld_ascale;      // B_MX: their row stride (bytes)
+  uint8_t* cscale;        // kEpiGeluMx: output E8M0 scales (M, N/32); C holds the codes
+  int64_t ld_cscale;
+  int M, N, K;         // split-K: K is the per-split depth
+  int tiles_m, tiles_n;
+  // 8-wave bias epilogue: per-row sums of squares of the bf16 outputs of
+  // columns [0, ss_cols), one fp32 partial per 64-column slice at
+  // rowss[row * ld_rowss + col / 64] (null: none)
+  float* rowss = nullptr;
+  int64_t ld_rowss = 0;
+  int ss_cols = 0;
+};
+
+// EPI value of the split-K pass: the accumulators go to the fp32 partial
+// buffer as they are, the epilogue runs in splitk_epilogue_kernel.
+constexpr int kEpiPartial = 16;
+// EPI value of the MX kernel's FF up-projection: the GELU epilogue whose
+// bf16 result leaves as MXFP8 rows (codes in C, E8M0 scales in cscale) --
+// the next product's quantised activations, written by this one.
+constexpr int kEpiGeluMx = 5;
+constexpr int kGroupM = 4;
+
+__device__ __forceinline__ void tile_coords(int bid, int nblocks, int tiles_m, int tiles_n, int& tm,
+                                            int& tn) {
+  // XCD-contiguous renumbering: hardware sends block b to XCD b % 8.
+  const int q = nblocks / kNumXcd, r = nblocks % kNumXcd;
+  const int xcd = bid % kNumXcd, idx = bid / kNumXcd;
+  const int logical = xcd * q + (xcd < r ? xcd : r) + idx;
+  // grouped ordering: kGroupM tile-rows sweep the tile-columns together
+  const int per_group = kGroupM * tiles_n;
+  const int group = logical / per_group;
+  const int first_m = group * kGroupM;
+  const int gsize = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
+  const int in_group = logical % per_group;
+  tm = first_m + in_group % gsize;
+  tn = in_group / gsize;
+}
+
+// f(integral_constant<int, I>) for I = I0 .. N-1, in order
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
+// 16-byte chunk XOR of row r in the 8-wave kernels' stages, 64-byte rows (4
+// chunks) and 128-byte rows (8 chunks).  ds_read_b128 services a wave's lanes
+// 16 at a time, in the lane-octet pairs (0, 3), (1, 2), (4, 7), (5, 6)
+// (probed: two octets reading the same banks at other addresses conflict only
+// in those pairs), and its conflicts were probed per read pattern (rocprofv3
+// SQ_LDS_BANK_CONFLICT of a one-read kernel over 290 lane -> address tables):
+// the 32x32 fragment reads (lane = row 0-31, lane / 32 = chunk half) are
+// conflict-free under chunk ^ ((r / 4) % 4) and chunk ^ ((r / 2) % 8), but the
+// 16x16 reads (lane % 16 = row, lane / 16 = chunk quarter) conflict under
+// those (the FF up-projection: 36-39 M conflict cycles per launch) and not
+// under chunk ^ (r bit 0 | r bit 2 << 1) and chunk ^ (r bit 1 | r bit 0 << 1
+// | r bit 2 << 2).
+__device__ __forceinline__ int g8_swz64(int r, bool s16) { return s16 ? ((r & 1) | ((r >> 1) & 2)) : ((r >> 2) & 3); }
+__device__ __forceinline__ int g8_swz128(int r, bool s16) {
+  return s16 ? (((r >> 1) & 1) | ((r & 1) << 1) | (r & 4)) : ((r >> 1) & 7);
+}
+
+// gemm_kg.hip: launch the mid-size kernel with BM-row tiles (64, 128 or 192)
+// and `splits` K ranges (epi kEpiPartial; p.K is then the depth of one).
+// The caller has checked kg_ok.  False: no such kernel.
+bool kg_launch(int bkind, const GemmArgs& p, int epi, int bm, int splits, hipStream_t s);
 
 }  // namespace ltx

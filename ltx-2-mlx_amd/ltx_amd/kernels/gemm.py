@@ -24,6 +24,7 @@ activations' E4M3 rounding moves outputs by a few percent of their range.
 
 from __future__ import annotations
 
+import functools
 import os
 from dataclasses import dataclass
 
@@ -143,27 +144,14 @@ def dequantize(weight: LinearWeight) -> torch.Tensor:
     return out
 
 
-# Block budget of an automatic split-K launch (128x128 tiles x splits).
-SPLITK_MAX_BLOCKS = 80
+_WFORMAT = {"bf16": 0, "int8": 1, "mxfp8": 2}
 
 
-def auto_splits(m: int, n: int, k: int, kind: str, max_blocks: int | None = None) -> int:
-    """Split-K factor for a few-row product: the largest power of two keeping
-    at most ``max_blocks`` (default ``SPLITK_MAX_BLOCKS``) blocks of 128x128
-    tiles, at least 256 of K per split and K divisible by the split
-    granularity; 1 when the product already fills the chip (or has more than
-    256 rows)."""
-    max_blocks = SPLITK_MAX_BLOCKS if max_blocks is None else max_blocks
-    if m > 256 or k < 1024:
-        return 1
-    tiles = ((m + 127) // 128) * ((n + 127) // 128)
-    if tiles >= 160:
-        return 1
-    unit = 128 if kind == "mxfp8" else 64
-    s = 1
-    while tiles * s * 2 <= max_blocks and k % (unit * s * 2) == 0 and k // (s * 2) >= 256:
-        s *= 2
-    return s
+@functools.lru_cache(maxsize=4096)
+def auto_splits(m: int, n: int, k: int, kind: str) -> int:
+    """Split-K factor of a product whose output tiles leave CUs idle, from the
+    library's cost model (ltx_gemm_auto_splits); 1 when one pass is as fast."""
+    return _lib.lib().ltx_gemm_auto_splits(m, n, k, _WFORMAT.get(kind, -1))
 
 
 # Few-row products (at most ROWS_MAX_M rows: the 68 / 121-token audio stream)
@@ -428,7 +416,7 @@ def linear_rowss(x: torch.Tensor, weight: LinearWeight, ss_cols: int, *,
         flags |= _lib.GEMM_ROUND_THEN_BIAS
     sig = n if sigmoid_from is None else int(sigmoid_from)
     bptr = None if weight.bias is None else weight.bias.data_ptr()
-    fmt = {"bf16": 0, "int8": 1, "mxfp8": 2}[weight.kind]
+    fmt = _WFORMAT[weight.kind]
     sptr, lds = (None, 0) if weight.kind == "bf16" else (
         weight.scale.data_ptr(), weight.scale.stride(0) if weight.kind == "mxfp8" else 0)
     hook = LAUNCH_HOOK
@@ -454,8 +442,8 @@ def linear(x: torch.Tensor, weight: LinearWeight, *, epilogue: int = EPI_BIAS,
     (N) are required; ``out`` may be ``residual`` itself (in-place update).
     With ``EPI_BIAS``, columns ``n >= sigmoid_from`` get the 2*sigmoid head
     gate instead (fused gate-logit columns of a Q/QKV projection).
-    ``splits``: split-K factor (None: ``auto_splits`` for the 128x128 tiles,
-    1: single pass); the split form sums fp32 partials from a workspace.
+    ``splits``: split-K factor (None: ``auto_splits`` with the automatic tile
+    choice, 1: single pass); the split form sums fp32 partials from a workspace.
     With ``ROWS_KERNEL`` set, few-row products with ``splits=None`` and the
     automatic tile choice run on :func:`linear_rows`.
     """
@@ -509,7 +497,7 @@ def linear(x: torch.Tensor, weight: LinearWeight, *, epilogue: int = EPI_BIAS,
     hook = LAUNCH_HOOK
     info = (weight.kind, m, n, k, epilogue) if hook is not None else None
     if splits is None:
-        splits = auto_splits(m, n, k, weight.kind) if tile in (TILE_AUTO, TILE_128) else 1
+        splits = auto_splits(m, n, k, weight.kind) if tile == TILE_AUTO else 1
     if hook is not None:
         hook("pre", info)
     if splits == 1 and _mx_eligible(m, n, k, weight, tile):
