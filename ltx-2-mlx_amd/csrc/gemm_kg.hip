@@ -17,11 +17,18 @@
 //
 // Units reach LDS by direct buffer loads into rings several units deep; the
 // fragments of the next k-step are read while the MFMAs of the current one
-// run, also across the one barrier per unit.  What bounds it: a 128 x 128
-// tile asks 384 (8-bit weights) or 512 (bf16) operand bytes per k of its CU
-// for 8 cycles of MFMA per k, against the 64 bytes per cycle that an L2
-// serves each CU: bf16 tiles of 128 rows run at the L2's limit, the others
-// at the issue of MFMAs, fragment reads and conversions.
+// run, also across the one barrier per unit.  Every row piece that a load
+// moves is a whole 128-byte line: both groups' 64-byte halves lie in one LDS
+// row.  (With a row of 64 bytes per group each line took two requests, and
+// the requests bounded the bf16 tiles: 384 x 4096 -> 4096 36.5 -> 30.2 us,
+// 384 x 4096 -> 16384 69.4 -> 59.3, 384 x 16384 -> 4096 105 -> 88, 1024 x
+// 16384 -> 4096 164 -> 144; 8-bit weights, whose activations were whole
+// lines already: 256 x 4096 -> 8192 MXFP8 27.1 -> 25.5, the rest within 3 %.)
+// What bounds it: a CU's operand bytes.  One CU streams at most 55-60 bytes
+// per ns of weights that come from HBM, however deep the ring (64-144 KB in
+// flight measured alike; 40 in 64-byte pieces), and ~110 of what the caches
+// hold, against a 128 x 128 tile's 384 (8-bit weights) or 512 (bf16) bytes
+// per k for 8 cycles of MFMA.
 #include "gemm_common.h"
 
 namespace ltx {
@@ -38,8 +45,8 @@ struct KgCfg {
   static constexpr int WM = BM / 2, WN = 64;         // wave tile
   static constexpr int AM = WM / 16, AN = WN / 16;   // its 16x16 accumulator blocks
   static constexpr int HM = AM / 2;                  // row blocks kept per group after the exchange
-  static constexpr int A_ROWB = 2 * KU, B_ROWB = 64; // LDS row bytes of a stage
-  static constexpr int A_BYTES = BM * A_ROWB, B_BYTES = BN * B_ROWB;  // one group's stage
+  static constexpr int A_ROWB = 128, B_ROWB = 128;   // LDS row bytes
+  static constexpr int A_BYTES = BM * 2 * KU, B_BYTES = BN * KU * ES;  // one group's stage
   // ring depths in units.  192-row tiles of 8-bit weights: three whole units
   // exceed the LDS, so the activations (mostly L2 hits) run one unit ahead
   // and the weights (HBM) two.
@@ -73,6 +80,12 @@ struct KgCfg {
   static_assert(!MXS || RA <= 4, "a scale load lands within the four units before its use");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS");
 };
+
+// 16-byte chunk XOR of a 128-byte row that holds both groups' halves, read as
+// chunk 4 grp + q of rows r16: a lane-octet pair that ds_read_b128 serves
+// together (see g8_swz128) holds eight rows at q and eight at q ^ 1, and even
+// rows keep chunk bit 0, so the pair covers all 64 banks.
+__device__ __forceinline__ int kg_swz_pair(int r) { return r & 6; }
 
 // 4-byte direct load: one dword per lane to lds_dst + 4 * lane
 __device__ __forceinline__ void kg_dma4(const void* base, int num_records, uint32_t voff, int soff, char* lds_dst) {
@@ -111,30 +124,32 @@ __global__ __launch_bounds__(kKgThreads, 1) void gemm_kg_kernel(GemmArgs p) {
   const int live = __builtin_amdgcn_readfirstlane((m0 + wm * WM < p.M && n0 + wn * WN < p.N) ? 1 : 0);
 
   // ---- direct-load sources: instruction d of wave w fills 1 KiB block
-  // 8 d + w of the unit (group 0's stage, then group 1's); lane j its 16-byte
-  // slot j, which holds the logical chunk that the row's XOR swizzle puts
-  // there (conflict-free for the 16x16 fragment reads).  Rows past M / N
+  // 8 d + w of the unit, 8 LDS rows of 128 bytes; lane j its 16-byte slot j,
+  // which holds the logical chunk that the row's XOR swizzle puts there.
+  // Rows of 64 bytes per group (weights; bf16 weights' activations) hold both
+  // groups' halves, so every row of a load is a whole 128-byte line: half
+  // lines cost the L2 as many requests each.  8-bit weights' activations, 128
+  // bytes per group, are group 0's rows, then group 1's.  Rows past M / N
   // re-read the last row; the record counts bound every load to its operand.
   const int a_records = (int)((int64_t)p.M * p.lda * 2), b_records = (int)((int64_t)p.N * p.ldb * ES);
   uint32_t a_src[A_DMA];
 #pragma unroll
   for (int d = 0; d < A_DMA; ++d) {
-    constexpr int BLK = A_BYTES / 1024;
-    const int j = 8 * d + wave, g = j / BLK, blk = j % BLK;
-    const int r = A_ROWB == 128 ? 8 * blk + (lane >> 3) : 16 * blk + (lane >> 2);
-    const int chunk = A_ROWB == 128 ? (lane & 7) ^ g8_swz128(r, true) : (lane & 3) ^ g8_swz64(r, true);
+    const int lr = 8 * (8 * d + wave) + (lane >> 3);  // LDS row
+    const int r = BF ? lr : lr % BM, g = BF ? 0 : lr / BM;
+    const int chunk = (lane & 7) ^ (BF ? kg_swz_pair(r) : g8_swz128(r, true));
     int gm = m0 + r;
     gm = gm < p.M ? gm : p.M - 1;
-    a_src[d] = (uint32_t)(((int64_t)gm * p.lda + k0) * 2) + g * A_ROWB + chunk * 16;
+    a_src[d] = (uint32_t)(((int64_t)gm * p.lda + k0) * 2) + g * 128 + chunk * 16;
   }
   uint32_t b_src[B_DMA];
 #pragma unroll
   for (int d = 0; d < B_DMA; ++d) {
-    const int r = 16 * wave + (lane >> 2);  // block 8 d + wave: group d
-    const int chunk = (lane & 3) ^ g8_swz64(r, true);
+    const int r = 8 * (8 * d + wave) + (lane >> 3);
+    const int chunk = (lane & 7) ^ kg_swz_pair(r);
     int gn = n0 + r;
     gn = gn < p.N ? gn : p.N - 1;
-    b_src[d] = (uint32_t)(((int64_t)gn * p.ldb + k0) * ES) + d * B_ROWB + chunk * 16;
+    b_src[d] = (uint32_t)(((int64_t)gn * p.ldb + k0) * ES) + chunk * 16;
   }
   // MXFP8 scales, four units at a time: 16 bytes per weight row, a dword per
   // lane of 16 rows per wave (a dword per unit of 64 rows per wave would
@@ -158,24 +173,24 @@ __global__ __launch_bounds__(kKgThreads, 1) void gemm_kg_kernel(GemmArgs p) {
   auto load = [&](int u, int sa, int sb, int l) __attribute__((always_inline)) {
     const int ua = u + RA < KT ? u + RA : KT - 1, ub = u + RB < KT ? u + RB : KT - 1;
     if (l < A_DMA)
-      buffer_dma16(p.A, a_records, a_src[l < A_DMA ? l : 0], ua * 2 * A_ROWB,
+      buffer_dma16(p.A, a_records, a_src[l < A_DMA ? l : 0], ua * 4 * Cfg::KU,
                    lds + sa * 2 * A_BYTES + (8 * l + wave) * 1024);
     else
-      buffer_dma16(p.B, b_records, b_src[l >= A_DMA ? l - A_DMA : 0], ub * 2 * B_ROWB,
+      buffer_dma16(p.B, b_records, b_src[l >= A_DMA ? l - A_DMA : 0], ub * 2 * Cfg::KU * ES,
                    lds + Cfg::B_OFF + sb * 2 * B_BYTES + (8 * (l - A_DMA) + wave) * 1024);
   };
 
   // ---- fragment addresses of the lane (row r16 of a 16-row block, k-quarter
   // q) in unit slot 0.  8-bit codes: k-step s is k = 16 q + 8 s + [0, 8) in
-  // both operands (codes: chunk q of the 64-byte row; activations: chunk
+  // both operands (codes: chunk q of the group's half row; activations: chunk
   // 2 q + s of the 128-byte row); bf16: k = 8 q + [0, 8).
   const int r16 = lane & 15, q = lane >> 4;
   int a_rd[Cfg::KS];
 #pragma unroll
   for (int s = 0; s < Cfg::KS; ++s)
-    a_rd[s] = grp * A_BYTES + (wm * WM + r16) * A_ROWB +
-              (BF ? (q ^ g8_swz64(r16, true)) * 16 : ((2 * q + s) ^ g8_swz128(r16, true)) * 16);
-  const int w_rd = Cfg::B_OFF + grp * B_BYTES + (wn * WN + r16) * B_ROWB + (q ^ g8_swz64(r16, true)) * 16;
+    a_rd[s] = (wm * WM + r16) * A_ROWB + (BF ? ((4 * grp + q) ^ kg_swz_pair(r16)) * 16
+                                             : grp * A_BYTES + ((2 * q + s) ^ g8_swz128(r16, true)) * 16);
+  const int w_rd = Cfg::B_OFF + (wn * WN + r16) * B_ROWB + ((4 * grp + q) ^ kg_swz_pair(r16)) * 16;
   const int s_rd = Cfg::SC_OFF + (wn * WN + r16) * 16 + 2 * grp + (q >> 1);  // the lane's k-block of 32
 
   float s_i8[AN];
