@@ -686,8 +686,10 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_kernel(GemmArgs p) {
 // 48 KB stages of bf16 activations (256 x 128 B) and raw weight codes
 // (256 x 64 B).  The MXFP8 / int8 codes are dequantised per fragment with the
 // exact format arithmetic, so the bf16 MFMA sees bit-exact weights.  bf16
-// weights: five 32 KB stages of 32-deep bf16 rows of both operands, the
-// direct loads four stages ahead, 32 MFMAs per cluster, no dequantisation.
+// weights: 32-deep stages that reach LDS in pairs (128-byte rows of both
+// operands), 32 MFMAs per cluster, no dequantisation; 64-byte rows, twice the
+// L2 requests, measured 390 against 350 us on FF up at M = 3456, 294 against
+// 267 on QKV, 228 against 200 on 2048 x 4096 -> 16384.
 // MX (8-bit codes of both operands): 16 scaled 32x32x64 MFMAs per cluster.
 //
 // Inside a stage the k order of the MFMA slots is permuted so that a lane
@@ -697,20 +699,21 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_kernel(GemmArgs p) {
 // scaled MFMA, lane half h, k = 32p + 16h + [0, 16).  The sum over the stage
 // is the same set of products.
 constexpr int kG8Threads = 512;
-// the automatic tile choice uses the 8-wave kernel for 8-bit weights (MXFP8
-// and int8) on problems of at least 100 256x256 tiles, and for bf16 weights on
-// problems of at least 160
+// the automatic tile choice uses the 8-wave kernel from 100 256x256 tiles on
 
-template <int BKIND, int BM_ = 256, int BF_STAGES = 5>
+template <int BKIND, int BM_ = 256>
 struct G8Cfg {
   static constexpr bool MX = BKIND == B_MX;
-  // bf16 weights: a 64-deep stage of both bf16 operands (64 KB) leaves room
-  // for only two stages, so the stages are 32 deep (64-byte rows of both
-  // operands, laid out like the 8-bit code rows) in a ring of BF_STAGES, the
-  // direct loads running BF_STAGES - 1 stages ahead
+  // bf16 weights: stages are 32 deep, but both operands reach LDS in pairs of
+  // stages, rows of 128 bytes: a 64-byte piece costs the L2 a request like a
+  // whole line does, and at two per line the requests kept its channels 0.7
+  // busy.  Rings of A_PAIRS and B_PAIRS pairs -- all that 160 KB hold: the
+  // activations (mostly L2 hits) one pair ahead, the weights (HBM) two.
   static constexpr bool BF = BKIND == B_BF16;
   static constexpr int BM = BM_, BN = 256, BK = BF ? 32 : 64;
-  static constexpr int STAGES = BF ? BF_STAGES : 3;
+  static constexpr int A_PAIRS = BM == 256 ? 2 : 3, B_PAIRS = 3;
+  // stages of one turn of the rings (bf16: of both), the loop's unrolling
+  static constexpr int STAGES = BF ? (A_PAIRS == 2 ? 12 : 6) : 3;
   // 128x64 wave tiles: each weight fragment is dequantised by the two waves
   // that share its columns rather than four (64x128 tiles read fewer LDS
   // bytes per MFMA, but MXFP8 measured 2.5 % slower with them: the
@@ -729,13 +732,13 @@ struct G8Cfg {
   static constexpr int TM16 = WM / 16, TN16 = WN / 16;
   // bf16 activations (MX: 8-bit codes like the weights), 8-bit weight codes
   // (BF: bf16 weights)
-  static constexpr int A_ROWB = MX ? BK : BK * 2, B_ROWB = BF ? BK * 2 : BK;
+  // (BF: a pair of stages)
+  static constexpr int A_ROWB = MX ? BK : 128, B_ROWB = BF ? 128 : BK;
   static constexpr int A_BYTES = BM * A_ROWB, B_BYTES = BN * B_ROWB;
-  static constexpr int STAGE = A_BYTES + B_BYTES;
   // LDS: the A stages, then the B stages (every fragment read is then a fixed
   // per-lane register plus an immediate offset below 64 KiB)
-  static constexpr int B_REGION = STAGES * A_BYTES;
-  static constexpr int A_DMA = A_BYTES / 1024 / 8, B_DMA = B_BYTES / 1024 / 8;  // per wave per stage
+  static constexpr int B_REGION = (BF ? A_PAIRS : STAGES) * A_BYTES;
+  static constexpr int A_DMA = A_BYTES / 1024 / 8, B_DMA = B_BYTES / 1024 / 8;  // per wave per stage (BF: pair)
   // epilogue staging rows: 16x16 accumulators, 128-byte rows with their
   // 16-byte chunks XORed by (row / 2) % 8 (conflict-free for both the 8-byte
   // accumulator writes and the 16-byte row reads, probed); 32x32 (MX), rows
@@ -747,7 +750,7 @@ struct G8Cfg {
   // the column values (bias, gate) follow the epilogue's staging area; they
   // are written after the main loop, so they may lie inside the stage ring
   static constexpr int COL_OFF = EPI_BYTES;
-  static constexpr int RING = STAGES * STAGE;
+  static constexpr int RING = B_REGION + (BF ? B_PAIRS : STAGES) * B_BYTES;
   static constexpr bool COL_IN_RING = COL_OFF < RING;
   static constexpr int LDS_BYTES = (RING > EPI_BYTES + COL_BYTES) ? RING : EPI_BYTES + COL_BYTES;
   // MXFP8 scales of eight stages (256 rows x 16 E8M0 bytes), double buffered;
@@ -776,6 +779,7 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   constexpr bool MX = Cfg::MX, BF = Cfg::BF, S16 = Cfg::S16;
   constexpr int TM16 = Cfg::TM16, TN16 = Cfg::TN16;
   constexpr int STAGES = Cfg::STAGES, AHEAD = STAGES - 1;
+  constexpr int AP = Cfg::A_PAIRS, BP = Cfg::B_PAIRS;
   __shared__ __attribute__((aligned(1024))) char lds[Cfg::TOTAL];
 
   const int tid = threadIdx.x;
@@ -804,8 +808,8 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // block of LDS, lane j its 16-byte slot j; the lane's source address picks
   // the logical chunk that the slot holds under the XOR swizzle of its row
   // (g8_swz128 for the 128-byte A rows, 8 per block; g8_swz64 for the 64-byte
-  // rows, 16 per block), the one under which this kernel's fragment reads are
-  // conflict-free.  Rows past M / N re-read the last row.
+  // rows, 16 per block; swz_pair for BF's rows of a stage pair), the one under
+  // which this kernel's fragment reads are conflict-free.  Rows past M / N re-read the last row.
   // Direct loads as buffer loads: a buffer descriptor per operand (scalar
   // registers), a fixed 32-bit per-lane byte offset in one vector register,
   // the stage's advance as the scalar offset and the LDS destination in M0
@@ -817,31 +821,45 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   uint32_t a_src[A_DMA];
 #pragma unroll
   for (int d = 0; d < A_DMA; ++d) {
-    if constexpr (MX || BF) {
-      // activation codes (MX) or 32-deep bf16 rows (BF): 64-byte rows laid
-      // out like the weight codes
+    if constexpr (MX) {
+      // activation codes: 64-byte rows laid out like the weight codes
       const int r = 16 * (8 * d + wave) + (lane >> 2);
       int gm = m0 + r;
       gm = gm < p.M ? gm : p.M - 1;
       const int chunk = (lane & 3) ^ g8_swz64(r, S16);
-      a_src[d] = (uint32_t)((int64_t)gm * p.lda * (MX ? 1 : 2)) + chunk * 16;
+      a_src[d] = (uint32_t)((int64_t)gm * p.lda) + chunk * 16;
     } else {
       const int r = 8 * (8 * d + wave) + (lane >> 3);
       int gm = m0 + r;
       gm = gm < p.M ? gm : p.M - 1;
-      const int chunk = (lane & 7) ^ g8_swz128(r, S16);
+      const int chunk = (lane & 7) ^ (BF ? swz_pair(r) : g8_swz128(r, S16));
       a_src[d] = (uint32_t)((int64_t)gm * p.lda * 2) + chunk * 16;
     }
   }
   uint32_t b_src[B_DMA];
 #pragma unroll
   for (int d = 0; d < B_DMA; ++d) {
-    const int r = 16 * (8 * d + wave) + (lane >> 2);
+    const int r = BF ? 8 * (8 * d + wave) + (lane >> 3) : 16 * (8 * d + wave) + (lane >> 2);
     int gn = n0 + r;
     gn = gn < p.N ? gn : p.N - 1;
-    const int chunk = (lane & 3) ^ g8_swz64(r, S16);
+    const int chunk = BF ? (lane & 7) ^ swz_pair(r) : (lane & 3) ^ g8_swz64(r, S16);
     b_src[d] = (uint32_t)((int64_t)gn * p.ldb * (BF ? 2 : 1)) + chunk * 16;
   }
+  // BF: an operand's pair `pair` (clamped to the last one) into ring slot `slot`
+  const int last_pair = (KT >> 1) - 1;
+  auto dma_pair_a = [&](int pair, int slot) __attribute__((always_inline)) {
+    pair = pair < last_pair ? pair : last_pair;
+#pragma unroll
+    for (int d = 0; d < A_DMA; ++d)
+      buffer_dma16(p.A, a_records, a_src[d], pair * A_ROWB, lds + slot * A_BYTES + (8 * d + wave) * 1024);
+  };
+  auto dma_pair_b = [&](int pair, int slot) __attribute__((always_inline)) {
+    pair = pair < last_pair ? pair : last_pair;
+#pragma unroll
+    for (int d = 0; d < B_DMA; ++d)
+      buffer_dma16(p.B, b_records, b_src[d], pair * B_ROWB,
+                   lds + B_REGION + slot * B_BYTES + (8 * d + wave) * 1024);
+  };
   auto dma_stage = [&](int kt, int buf) __attribute__((always_inline)) {
     char* As = lds + buf * A_BYTES;
     char* Bs = lds + B_REGION + buf * B_BYTES;
@@ -867,8 +885,7 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   }
   // 16x16x32 fragments: lane (r16, q) = row r16 of a 16-row block, k-quarter
   // q.  Weights: one 16-byte read per block and stage, chunk q of the 64-byte
-  // row (8-bit codes: k = 16 q + [0, 16), both k-steps; BF: bf16 k = 8 q +
-  // [0, 8) of the 32-deep stage).  8-bit codes: k-step s of the stage is
+  // row (8-bit codes: k = 16 q + [0, 16), both k-steps).  8-bit codes: k-step s of the stage is
   // k = 16 q + 8 s + [0, 8) in lane q for both operands -- the activation
   // fragment is chunk 2 q + s of the 128-byte row -- so the E8M0 block of a
   // lane's codes is q / 2 in both k-steps.  Every 16 lanes read 16
@@ -877,13 +894,17 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // The activation bases come as a low / high pair (stage buffers 0-1 / 1-2
   // of the 8-bit-code ring) so that the offsets fit the 16-bit immediate.
   const int r16 = lane & 15, q = lane >> 4;
+  // BF: chunk 4 s + q of the 128-byte row of a pair is the lane's fragment of
+  // its stage s; the weights' bases as a low / high pair too (slots 0 and 1-2).
   const int w16 = B_REGION + (wn * WN + r16) * B_ROWB + ((q ^ g8_swz64(r16, true)) * 16);
-  int x16_lo[2], x16_hi[2];
+  int x16_lo[2], x16_hi[2], w16_lo[2], w16_hi[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    x16_lo[s] = BF ? (wm * WM + r16) * A_ROWB + ((q ^ g8_swz64(r16, true)) * 16)
-                   : (wm * WM + r16) * A_ROWB + (((2 * q + s) ^ g8_swz128(r16, true)) * 16);
+    const int pair_chunk = ((4 * s + q) ^ swz_pair(r16)) * 16;
+    x16_lo[s] = (wm * WM + r16) * A_ROWB + (BF ? pair_chunk : ((2 * q + s) ^ g8_swz128(r16, true)) * 16);
     x16_hi[s] = x16_lo[s] + A_BYTES;
+    w16_lo[s] = B_REGION + (wn * WN + r16) * B_ROWB + pair_chunk;
+    w16_hi[s] = w16_lo[s] + B_BYTES;
   }
   // MXFP8 scales reach LDS by direct loads too, eight stages at a time: the
   // loop then holds no register-destined global load, whose first use would
@@ -967,6 +988,15 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
         for (int i = 0; i < TM; ++i)
           fa8[pp][i] = *reinterpret_cast<const u32x4*>(lds + a_mx[pp] + BUF * A_BYTES + i * 32 * A_ROWB);
       }
+    } else if constexpr (BF) {
+      // BUF = kt % STAGES: pair BUF / 2 in slots BUF / 2 % AP and % BP
+      constexpr int SA = BUF / 2 % AP, SB = BUF / 2 % BP, S = BUF & 1;
+      const int wb = SB == 0 ? w16_lo[S] : w16_hi[S] + (SB - 1) * B_BYTES;
+      const int xb = SA == 0 ? x16_lo[S] : x16_hi[S] + (SA - 1) * A_BYTES;
+#pragma unroll
+      for (int jb = 0; jb < TN16; ++jb) w16f[jb] = *reinterpret_cast<const u32x4*>(lds + wb + jb * 16 * B_ROWB);
+#pragma unroll
+      for (int ib = 0; ib < TM16; ++ib) x16f[0][ib] = *reinterpret_cast<const bf16x8*>(lds + xb + ib * 16 * A_ROWB);
     } else {
 #pragma unroll
       for (int jb = 0; jb < TN16; ++jb)
@@ -1094,14 +1124,23 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
 
   // ---- prologue: scales of octet 0, stages 0 .. AHEAD-1 in flight, then one
   // barrier for all waves
-  dma_scales(0);
-  dma_stage(0, 0);
-  if (KT > 1) dma_stage(1, 1);
-  static_for<2, AHEAD>([&](auto ic) {
-    if (KT > decltype(ic)::value) dma_stage(decltype(ic)::value, decltype(ic)::value);
-  });
-  wait_vmcnt<0>();
-  __syncthreads();
+  // BF: pairs in flight when pair b's loads must have landed -- those of the
+  // AP - 2 activation pairs and of the one weight pair after it
+  constexpr int BF_FLIGHT = (AP - 2) * A_DMA + B_DMA;
+  if constexpr (BF) {
+    dma_pair_a(0, 0);
+    dma_pair_b(0, 0);
+    if constexpr (AP == 3) dma_pair_a(1, 1);
+    dma_pair_b(1, 1);
+    wait_vmcnt<BF_FLIGHT>();
+    barrier_nofence();
+  } else {
+    dma_scales(0);
+    dma_stage(0, 0);
+    if (KT > 1) dma_stage(1, 1);
+    wait_vmcnt<0>();
+    __syncthreads();
+  }
   if (grp == 1) barrier_nofence();  // group 1 runs half a stage behind
 
   // Clusters are whole stages.  Stage s is first read by group 0's memory
@@ -1114,22 +1153,35 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // direct loads re-read stage KT-1 into the buffer nobody reads any more,
   // so every stage issues the same loads and the waits are exact.  The scales
   // of octet o+1 go out (group 0) with stage 8o's loads.
-  // SUB = kt % 8 (compile-time in the unrolled loop).
+  // BF: the memory cluster of a pair's first stage issues the activations'
+  // next free pair, that of its second stage the weights'; only the last
+  // stage of a pair waits, for the next pair.
   // The loop is compiled once per group (GRP), so the group-specific waits
   // and scale loads are resolved at compile time.
   auto stage_iter = [&](int kt, auto bufc, auto grpc) __attribute__((always_inline)) {
     constexpr int BUF = decltype(bufc)::value;
     constexpr int GRP = decltype(grpc)::value;
     const bool oct_start = SCALED && (kt & 7) == 0;
+    constexpr bool PAIR_END = (BUF & 1) != 0;
     // memory cluster (MX: group 1 moves the activations' scale octets)
-    if ((GRP == 0 || MX) && oct_start) dma_scales((kt >> 3) + 1);
-    dma_stage(kt + AHEAD < KT ? kt + AHEAD : KT - 1, (BUF + AHEAD) % STAGES);
+    if constexpr (BF) {
+      if (PAIR_END) dma_pair_b((kt >> 1) + BP - 1, (BUF / 2 + BP - 1) % BP);
+      else dma_pair_a((kt >> 1) + AP - 1, (BUF / 2 + AP - 1) % AP);
+    } else {
+      if ((GRP == 0 || MX) && oct_start) dma_scales((kt >> 3) + 1);
+      dma_stage(kt + AHEAD < KT ? kt + AHEAD : KT - 1, (BUF + AHEAD) % STAGES);
+    }
     if (live) read_stage(kt, bufc);
     wait_lgkmcnt0();
     if (live) prep_stage(kt);
     if (GRP == 1) {
-      if (MX && oct_start) wait_vmcnt<VM_DMA + VM_SCALES>();
-      else wait_vmcnt<(AHEAD - 1) * VM_DMA>();
+      if constexpr (BF) {
+        if (PAIR_END) wait_vmcnt<BF_FLIGHT>();
+      } else if (MX && oct_start) {
+        wait_vmcnt<VM_DMA + VM_SCALES>();
+      } else {
+        wait_vmcnt<VM_DMA>();
+      }
     }
     barrier_nofence();
     // compute cluster
@@ -1137,13 +1189,18 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
     if (live) compute_stage(kt);
     __builtin_amdgcn_s_setprio(0);
     if (GRP == 0) {
-      if (oct_start) wait_vmcnt<VM_DMA + VM_SCALES>();
-      else wait_vmcnt<(AHEAD - 1) * VM_DMA>();
+      if constexpr (BF) {
+        if (PAIR_END) wait_vmcnt<BF_FLIGHT>();
+      } else if (oct_start) {
+        wait_vmcnt<VM_DMA + VM_SCALES>();
+      } else {
+        wait_vmcnt<VM_DMA>();
+      }
     }
     barrier_nofence();
   };
-  // the loop unrolled over one turn of the ring, then the remainder (stage
-  // kt + i sits in buffer i)
+  // the loop unrolled over one turn of the rings, then the remainder (stage
+  // kt + i sits in buffer i; BF: i / 2 counts pairs)
   auto main_loop = [&](auto grpc) __attribute__((always_inline)) {
     int kt = 0;
     for (; kt + STAGES - 1 < KT; kt += STAGES)
@@ -1399,8 +1456,8 @@ static bool kg_ok(int bkind, int64_t M, int64_t N, int64_t Ks, int64_t lda, int6
 }
 
 // Modelled time (us) of a product on the mid-size kernel.  A round of one
-// workgroup per CU costs `unit` us per 128 k (measured alone at K = 4096,
-// tiles of 64 / 128 / 192 rows, one partial round), and however many rounds,
+// workgroup per CU costs `unit` us per 128 k (measured at K = 4096-8192,
+// tiles of 64 / 128 / 192 rows, weights from HBM), and however many rounds,
 // the L2s deliver about 13 TB/s of tile operands to the CUs (every shape with
 // all CUs busy measured 11-15 TB/s); 4 us of launch, first loads and
 // epilogue; split-K adds its second launch and one write and read of the fp32
@@ -1409,7 +1466,7 @@ static bool kg_ok(int bkind, int64_t M, int64_t N, int64_t Ks, int64_t lda, int6
 // 201 / 193, 220 / 197; 204 x 8192 -> 2048 64 rows, 1 / 2 / 4 splits
 // 39 / 27 / 20 against 32 / 24 / 19.
 static double kg_time(int bkind, int64_t M, int64_t N, int64_t K, int bm, int64_t splits) {
-  static const double unit_us[3][3] = {{0.70, 0.88, 1.05}, {0.87, 1.00, 1.25}, {0.55, 0.77, 1.02}};
+  static const double unit_us[3][3] = {{0.78, 1.08, 1.30}, {0.87, 1.00, 1.25}, {0.55, 0.77, 1.08}};
   const int64_t wgs = ((M + bm - 1) / bm) * ((N + 127) / 128) * splits;
   const double units = (double)(K / 128) / (double)splits;
   const double rounds = (double)((wgs + 255) / 256);
@@ -1439,7 +1496,10 @@ static int kg_rows(int bkind, int64_t M, int64_t N, int64_t K, int64_t splits, d
 // Whether an automatic launch takes the mid-size kernel: below 160 tiles of
 // 256x256 (from there the 256-row tiles fill the chip; 3456 x 4096 -> 4096 90
 // against 121 us), except where the 8-wave kernel's single round of 100-159
-// tiles models faster (2.1 us per 128 k measured; int8 2.4).
+// tiles models faster (2.1 us per 128 k measured; int8 2.4).  Measured, this
+// kernel against that one, K = 4096: 1728 x 4096 bf16 78 / 76, MXFP8 61 / 73;
+// 2048 x 4096 86 / 76, 67 / 77; 2304 x 4096 81 / 75, 81 / 75; 384 x 16384
+// 55 / 71, 51 / 76; 512 x 16384 93 / 77, 74 / 76; 700 x 12320 90 / 79, 86 / 77.
 static bool kg_auto(int bkind, const GemmArgs& p) {
   const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
   if (big >= 160 || !kg_ok(bkind, p.M, p.N, p.K, p.lda, p.ldb, p.ld_scale)) return false;
@@ -1473,15 +1533,11 @@ static int launch_epi_w(const GemmArgs& p, int tile, hipStream_t s) {
     // 61 us alone, but the step 1.0-1.6 ms slower in two A/B pairs -- 48 %
     // more CU time per launch, which the audio stream's work beside it then
     // lacks: explicit only, LTX_GEMM_TILE_G8_128.)
-    // bf16 weights (32-deep stages) take it where it measured faster at
-    // M = 3456 (16x16x32 MFMAs, one box): products at least as wide as deep
-    // (FF up 396 vs 422 us on the 4-wave kernel, QKV 291 vs 302, 4096^2 98.8
-    // vs 103.7, A2V out 57.5 vs 59.9) and the partial round of the A2V query
-    // projection (81 vs 87 us); the FF down product stays on the 4-wave
-    // kernel (393 vs 402 us).
+    // bf16 weights take it too: faster than the 4-wave kernel on every shape
+    // of 100 tiles on (FF up 350 vs 420 us, 4096^2 91 vs 105, FF down 339 vs
+    // 404, 1024 x 4096 -> 12320 87 vs 101).
     const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
-    const bool g8 = (BKIND == B_MXFP8 || BKIND == B_INT8 || (BKIND == B_BF16 && (p.N >= p.K || big < 160))) &&
-                    g8_ok<BKIND>(p);
+    const bool g8 = g8_ok<BKIND>(p);
     tile = big >= 160 ? (g8 ? 5 : 1) : (big >= 100 && g8 ? 5 : 2);
     // row sums of squares come from the 8-wave kernels' epilogues only
     if (p.rowss && tile != 5) tile = 5;

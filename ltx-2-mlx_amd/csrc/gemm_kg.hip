@@ -81,12 +81,6 @@ struct KgCfg {
   static_assert(LDS_BYTES <= 160 * 1024, "LDS");
 };
 
-// 16-byte chunk XOR of a 128-byte row that holds both groups' halves, read as
-// chunk 4 grp + q of rows r16: a lane-octet pair that ds_read_b128 serves
-// together (see g8_swz128) holds eight rows at q and eight at q ^ 1, and even
-// rows keep chunk bit 0, so the pair covers all 64 banks.
-__device__ __forceinline__ int kg_swz_pair(int r) { return r & 6; }
-
 // 4-byte direct load: one dword per lane to lds_dst + 4 * lane
 __device__ __forceinline__ void kg_dma4(const void* base, int num_records, uint32_t voff, int soff, char* lds_dst) {
   const __amdgpu_buffer_rsrc_t r =
@@ -137,7 +131,7 @@ __global__ __launch_bounds__(kKgThreads, 1) void gemm_kg_kernel(GemmArgs p) {
   for (int d = 0; d < A_DMA; ++d) {
     const int lr = 8 * (8 * d + wave) + (lane >> 3);  // LDS row
     const int r = BF ? lr : lr % BM, g = BF ? 0 : lr / BM;
-    const int chunk = (lane & 7) ^ (BF ? kg_swz_pair(r) : g8_swz128(r, true));
+    const int chunk = (lane & 7) ^ (BF ? swz_pair(r) : g8_swz128(r, true));
     int gm = m0 + r;
     gm = gm < p.M ? gm : p.M - 1;
     a_src[d] = (uint32_t)(((int64_t)gm * p.lda + k0) * 2) + g * 128 + chunk * 16;
@@ -146,7 +140,7 @@ __global__ __launch_bounds__(kKgThreads, 1) void gemm_kg_kernel(GemmArgs p) {
 #pragma unroll
   for (int d = 0; d < B_DMA; ++d) {
     const int r = 8 * (8 * d + wave) + (lane >> 3);
-    const int chunk = (lane & 7) ^ kg_swz_pair(r);
+    const int chunk = (lane & 7) ^ swz_pair(r);
     int gn = n0 + r;
     gn = gn < p.N ? gn : p.N - 1;
     b_src[d] = (uint32_t)(((int64_t)gn * p.ldb + k0) * ES) + chunk * 16;
@@ -188,9 +182,9 @@ __global__ __launch_bounds__(kKgThreads, 1) void gemm_kg_kernel(GemmArgs p) {
   int a_rd[Cfg::KS];
 #pragma unroll
   for (int s = 0; s < Cfg::KS; ++s)
-    a_rd[s] = (wm * WM + r16) * A_ROWB + (BF ? ((4 * grp + q) ^ kg_swz_pair(r16)) * 16
+    a_rd[s] = (wm * WM + r16) * A_ROWB + (BF ? ((4 * grp + q) ^ swz_pair(r16)) * 16
                                              : grp * A_BYTES + ((2 * q + s) ^ g8_swz128(r16, true)) * 16);
-  const int w_rd = Cfg::B_OFF + (wn * WN + r16) * B_ROWB + ((4 * grp + q) ^ kg_swz_pair(r16)) * 16;
+  const int w_rd = Cfg::B_OFF + (wn * WN + r16) * B_ROWB + ((4 * grp + q) ^ swz_pair(r16)) * 16;
   const int s_rd = Cfg::SC_OFF + (wn * WN + r16) * 16 + 2 * grp + (q >> 1);  // the lane's k-block of 32
 
   float s_i8[AN];
