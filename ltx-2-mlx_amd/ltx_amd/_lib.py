@@ -171,7 +171,16 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Handle of the current stream of t's device (the raw handle: building
+    torch's Stream object costs the host ~2 us per launch)."""
+    if not t.is_cuda:
+        raise ValueError(f"expected a device tensor, got one on {t.device}")
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+def flat(t: torch.Tensor) -> torch.Tensor:
+    """t with its elements in one dense run; t itself where it is dense."""
+    return t if t.is_contiguous() else t.reshape(-1).contiguous()
 
 
 def row_view(t: torch.Tensor, cols: int) -> tuple[torch.Tensor, int]:
@@ -179,6 +188,12 @@ def row_view(t: torch.Tensor, cols: int) -> tuple[torch.Tensor, int]:
     of unit column stride.  Copies only if the layout is not row-uniform."""
     if t.shape[-1] != cols:
         raise ValueError(f"last dim {t.shape[-1]} != {cols}")
+    st = t.stride()
+    if st[-1] == 1:  # the usual forms: rows of a matrix, or of one batch entry
+        if len(st) == 2:
+            return t, st[0]
+        if len(st) == 3 and t.shape[0] == 1:
+            return t, st[1]
     if t.dim() == 1:
         return t.contiguous(), cols
     if t.stride(-1) == 1:

@@ -145,8 +145,7 @@ def adaln_norm_fused(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tensor, 
     b, t, c = x.shape
     xv, xs = _lib.row_view(x, c)
     out = torch.empty((b, t, c), dtype=torch.bfloat16, device=x.device)
-    adaln_rows(xv, xs, scale.reshape(-1).contiguous(), shift.reshape(-1).contiguous(),
-               out, c, b * t, c, eps, 0)
+    adaln_rows(xv, xs, _lib.flat(scale), _lib.flat(shift), out, c, b * t, c, eps, 0)
     return out
 
 
@@ -195,5 +194,5 @@ def gated_add_fused(residual: torch.Tensor, branch: torch.Tensor, gate: torch.Te
     rv, rs = _lib.row_view(residual, c)
     bv, bs = _lib.row_view(branch, c)
     out = torch.empty((b, t, c), dtype=torch.bfloat16, device=residual.device)
-    gated_add_rows(rv, rs, bv, bs, gate.reshape(-1).contiguous(), out, c, b * t, c, 0)
+    gated_add_rows(rv, rs, bv, bs, _lib.flat(gate), out, c, b * t, c, 0)
     return out

@@ -481,10 +481,9 @@ def linear(x: torch.Tensor, weight: LinearWeight, *, epilogue: int = EPI_BIAS,
         if rv.data_ptr() != residual.data_ptr():
             raise ValueError("residual must be a row-strided view")
         rptr = rv.data_ptr()
-        g = gate.reshape(-1)
-        if g.dtype != torch.float32 or g.numel() != n:
+        if gate.dtype != torch.float32 or gate.numel() != n:
             raise ValueError("gate must be fp32 with N elements")
-        gate = g.contiguous()
+        gate = _lib.flat(gate)
         gptr = gate.data_ptr()
     flags = epilogue | (tile << 8)
     if weight.qlinear and weight.bias is not None:

@@ -112,8 +112,8 @@ class Attention:
                 buf, ss = gemm.linear_rowss(x, self.proj_q, inner, sigmoid_from=3 * inner)
             else:
                 buf = gemm.linear(x, self.proj_q, sigmoid_from=3 * inner)
-            q, k, v = buf[:, :inner], buf[:, inner:2 * inner], buf[:, 2 * inner:3 * inner]
-            g = buf[:, 3 * inner:3 * inner + gate_cols] if self.gated else None
+            q, k, v, g = buf.split((inner, inner, inner, buf.shape[1] - 3 * inner), 1)
+            g = None if not self.gated else (g if g.shape[1] == gate_cols else g[:, :gate_cols])
             k_tab = pe
         else:
             if fused:
