@@ -764,9 +764,12 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void flash_attn_kernel(
 
 // Combine of the split-KV partials: one thread per (query, head, 8 outputs).
 // O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s, m = max_s m_s; then the
-// same rounding and gate as the single-pass epilogue.
+// same rounding and gate as the single-pass epilogue.  Bound by the latency
+// of its loads: four splits' go out together (their sums stay in split order)
+// and one-wave workgroups spread a few queries over all CUs.
+constexpr int kCombineThreads = 64;
 template <int DH, bool GATED>
-__global__ __launch_bounds__(256) void attn_combine_kernel(SplitOut so, bf16* __restrict__ O, int64_t o_rs,
+__global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(SplitOut so, bf16* __restrict__ O, int64_t o_rs,
                                                            const bf16* __restrict__ G, int64_t g_rs,
                                                            int Tq, int H) {
   constexpr int CH = DH / 8;
@@ -776,22 +779,36 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(SplitOut so, bf16* __
   const int64_t qh = i / CH;  // q * H + head
   const int q = (int)(qh / H), head = (int)(qh % H);
   const int64_t plane = (int64_t)Tq * H;
+  constexpr int B = 4;
   float m = -INFINITY;
-  for (int sp = 0; sp < so.splits; ++sp) m = fmaxf(m, so.m[sp * plane + qh]);
+  for (int s0 = 0; s0 < so.splits; s0 += B) {
+    float ms[B];  // past the last split, its value again
+#pragma unroll
+    for (int u = 0; u < B; ++u) ms[u] = so.m[(s0 + u < so.splits ? s0 + u : so.splits - 1) * plane + qh];
+#pragma unroll
+    for (int u = 0; u < B; ++u) m = fmaxf(m, ms[u]);
+  }
   float l = 0.0f, o[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = 0.0f;
-  for (int sp = 0; sp < so.splits; ++sp) {
-    const float ms = so.m[sp * plane + qh];
-    const float w = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms - m);
-    l = fmaf(w, so.l[sp * plane + qh], l);
-    const float* src = so.o + (sp * plane + qh) * DH + c * 8;
-    const f32x4 a = *reinterpret_cast<const f32x4*>(src);
-    const f32x4 b = *reinterpret_cast<const f32x4*>(src + 4);
+  for (int s0 = 0; s0 < so.splits; s0 += B) {
+    float ms[B], ls[B];
+    f32x4 x[B][2];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o[e] = fmaf(w, a[e], o[e]);
-      o[4 + e] = fmaf(w, b[e], o[4 + e]);
+    for (int u = 0; u < B; ++u) {
+      const int64_t row = (s0 + u < so.splits ? s0 + u : so.splits - 1) * plane + qh;
+      ms[u] = so.m[row];
+      ls[u] = so.l[row];
+      x[u][0] = *reinterpret_cast<const f32x4*>(so.o + row * DH + c * 8);
+      x[u][1] = *reinterpret_cast<const f32x4*>(so.o + row * DH + c * 8 + 4);
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      if (s0 + u >= so.splits) break;
+      const float w = ms[u] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms[u] - m);
+      l = fmaf(w, ls[u], l);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = fmaf(w, x[u][e >> 2][e & 3], o[e]);
     }
   }
   const float inv_l = 1.0f / l;
@@ -1023,13 +1040,13 @@ static int launch_attn_splitkv(const void* Q, int64_t q_rs, const void* K, int64
                     (int)splits};
   const float scale_log2 = scale * 1.4426950408889634f;
   const int64_t cthreads = Tq * H * (head_dim / 8);
-  const int cblocks = (int)((cthreads + 255) / 256);
+  const int cblocks = (int)((cthreads + kCombineThreads - 1) / kCombineThreads);
 #define LTX_FAS(DH, G)                                                                              \
   do {                                                                                              \
     flash_attn_kernel<DH, false, kAttnSplitWaves, true, VROW><<<(int)nwg, 64 * kAttnSplitWaves, 0, s>>>( \
         (const bf16*)Q, q_rs, (const bf16*)K, k_rs, (const bf16*)V, v_ld, nullptr, 0, nullptr,      \
         0, (int)Tq, (int)Tk, (int)H, scale_log2, so, QNorm{});                                      \
-    attn_combine_kernel<DH, G><<<cblocks, 256, 0, s>>>(so, (bf16*)O, o_rs, (const bf16*)gate,       \
+    attn_combine_kernel<DH, G><<<cblocks, kCombineThreads, 0, s>>>(so, (bf16*)O, o_rs, (const bf16*)gate,       \
                                                        gate_rs, (int)Tq, (int)H);                    \
   } while (0)
   if (head_dim == 128) {
