@@ -673,8 +673,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_kernel(GemmArgs p) {
 // group 0 (waves 0-3) owns output rows 0-127 of the tile, group 1 (waves 4-7)
 // rows 128-255; wave w & 3 owns 64 output columns.  The groups run half a
 // stage apart: while one group issues its memory cluster (LDS fragment reads
-// of a stage, its share of the direct global->LDS loads two stages ahead, the
-// scale loads), the other group's compute cluster (the stage's 64 16x16x32
+// of a stage, its direct global->LDS loads of later stages, the scale loads), the other group's compute cluster (the stage's 64 16x16x32
 // MFMAs with the weight dequantisation of fragments 2-7 interleaved) keeps
 // the SIMD's matrix pipe busy.  The memory cluster ends, once its fragment
 // reads have landed, by decoding the stage's E8M0 scales and dequantising
@@ -682,9 +681,13 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_kernel(GemmArgs p) {
 // the barrier (FF up 402 -> 382 us: the dependent decode -> convert chain had
 // left the matrix pipe idle at the start of every compute cluster).
 // A workgroup barrier separates the clusters.  Both operands reach LDS by
-// global_load_lds (no staging registers, no LDS write instructions): three
-// 48 KB stages of bf16 activations (256 x 128 B) and raw weight codes
-// (256 x 64 B).  The MXFP8 / int8 codes are dequantised per fragment with the
+// direct loads (no staging registers, no LDS write instructions) of whole
+// 128-byte lines: stages of bf16 activations (256 x 128 B), moved by group 0
+// one stage ahead, and pairs of stages of raw weight codes (256 x 128 B),
+// moved by group 1 with the scales a pair ahead, two slots each (all that fits
+// beside the scales; against three single stages, 64 bytes of codes per row,
+// moved by all waves: FF up 331 -> 326 us, QKV 258 -> 252, 6144 x 4096 ->
+// 12320 438 -> 428, 3888 x 16384 -> 4096 349 -> 341).  The MXFP8 / int8 codes are dequantised per fragment with the
 // exact format arithmetic, so the bf16 MFMA sees bit-exact weights.  bf16
 // weights: 32-deep stages that reach LDS in pairs (128-byte rows of both
 // operands), 32 MFMAs per cluster, no dequantisation; 64-byte rows, twice the
@@ -711,9 +714,13 @@ struct G8Cfg {
   // activations (mostly L2 hits) one pair ahead, the weights (HBM) two.
   static constexpr bool BF = BKIND == B_BF16;
   static constexpr int BM = BM_, BN = 256, BK = BF ? 32 : 64;
-  static constexpr int A_PAIRS = BM == 256 ? 2 : 3, B_PAIRS = 3;
-  // stages of one turn of the rings (bf16: of both), the loop's unrolling
-  static constexpr int STAGES = BF ? (A_PAIRS == 2 ? 12 : 6) : 3;
+  // 8-bit weights (W8): the codes in pairs of 64-deep stages too (activation
+  // rows are 128 bytes as they are).  MX: single stages of both.
+  static constexpr bool W8 = !BF && !MX;
+  // ring slots: A stages (BF: pairs), B pairs (MX: stages)
+  static constexpr int A_SLOTS = MX ? 3 : (BM == 256 ? 2 : 3), B_SLOTS = W8 && BM == 256 ? 2 : 3;
+  // stages of one turn of both rings, the loop's unrolling
+  static constexpr int STAGES = MX ? 3 : (BF ? (BM == 256 ? 12 : 6) : (BM == 256 ? 4 : 6));
   // 128x64 wave tiles: each weight fragment is dequantised by the two waves
   // that share its columns rather than four (64x128 tiles read fewer LDS
   // bytes per MFMA, but MXFP8 measured 2.5 % slower with them: the
@@ -732,13 +739,16 @@ struct G8Cfg {
   static constexpr int TM16 = WM / 16, TN16 = WN / 16;
   // bf16 activations (MX: 8-bit codes like the weights), 8-bit weight codes
   // (BF: bf16 weights)
-  // (BF: a pair of stages)
-  static constexpr int A_ROWB = MX ? BK : 128, B_ROWB = BF ? 128 : BK;
+  // (BF: a pair of stages; W8: of the weights)
+  static constexpr int A_ROWB = MX ? BK : 128, B_ROWB = MX ? BK : 128;
   static constexpr int A_BYTES = BM * A_ROWB, B_BYTES = BN * B_ROWB;
   // LDS: the A stages, then the B stages (every fragment read is then a fixed
   // per-lane register plus an immediate offset below 64 KiB)
-  static constexpr int B_REGION = (BF ? A_PAIRS : STAGES) * A_BYTES;
-  static constexpr int A_DMA = A_BYTES / 1024 / 8, B_DMA = B_BYTES / 1024 / 8;  // per wave per stage (BF: pair)
+  static constexpr int B_REGION = A_SLOTS * A_BYTES;
+  // direct loads per wave and stage (BF: pair).  W8: group 0 moves the
+  // activations, group 1 the weights and scales, per wave and stage / pair
+  static constexpr int LOADERS = W8 ? 4 : 8;
+  static constexpr int A_DMA = A_BYTES / 1024 / LOADERS, B_DMA = B_BYTES / 1024 / LOADERS;
   // epilogue staging rows: 16x16 accumulators, 128-byte rows with their
   // 16-byte chunks XORed by (row / 2) % 8 (conflict-free for both the 8-byte
   // accumulator writes and the 16-byte row reads, probed); 32x32 (MX), rows
@@ -750,7 +760,7 @@ struct G8Cfg {
   // the column values (bias, gate) follow the epilogue's staging area; they
   // are written after the main loop, so they may lie inside the stage ring
   static constexpr int COL_OFF = EPI_BYTES;
-  static constexpr int RING = B_REGION + (BF ? B_PAIRS : STAGES) * B_BYTES;
+  static constexpr int RING = B_REGION + B_SLOTS * B_BYTES;
   static constexpr bool COL_IN_RING = COL_OFF < RING;
   static constexpr int LDS_BYTES = (RING > EPI_BYTES + COL_BYTES) ? RING : EPI_BYTES + COL_BYTES;
   // MXFP8 scales of eight stages (256 rows x 16 E8M0 bytes), double buffered;
@@ -776,10 +786,11 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   constexpr int A_DMA = Cfg::A_DMA, B_DMA = Cfg::B_DMA;
   constexpr int EPI_ROWB = Cfg::EPI_ROWB, EPI_WAVE = Cfg::EPI_WAVE;
   constexpr bool RESID = EPI == LTX_GEMM_EPI_RESIDUAL || EPI == LTX_GEMM_EPI_RESIDUAL_ROUND;
-  constexpr bool MX = Cfg::MX, BF = Cfg::BF, S16 = Cfg::S16;
+  constexpr bool MX = Cfg::MX, BF = Cfg::BF, W8 = Cfg::W8, S16 = Cfg::S16;
   constexpr int TM16 = Cfg::TM16, TN16 = Cfg::TN16;
-  constexpr int STAGES = Cfg::STAGES, AHEAD = STAGES - 1;
-  constexpr int AP = Cfg::A_PAIRS, BP = Cfg::B_PAIRS;
+  constexpr int STAGES = Cfg::STAGES;
+  constexpr int AP = Cfg::A_SLOTS, BP = Cfg::B_SLOTS;
+  constexpr int LOADERS = Cfg::LOADERS;
   __shared__ __attribute__((aligned(1024))) char lds[Cfg::TOTAL];
 
   const int tid = threadIdx.x;
@@ -817,7 +828,8 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // matrix-pipe slots from the other).  The descriptors' record counts bound
   // every load to its operand (g8_ok checks the 32-bit extents).
   const int a_records = (int)((int64_t)p.M * p.lda * (MX ? 1 : 2)),
-            b_records = (int)((int64_t)p.N * p.ldb * (BF ? 2 : 1));
+            b_records = (int)(((int64_t)(p.N - 1) * p.ldb + p.K) * (BF ? 2 : 1));
+  const int loader = W8 ? wave & 3 : wave;
   uint32_t a_src[A_DMA];
 #pragma unroll
   for (int d = 0; d < A_DMA; ++d) {
@@ -829,7 +841,7 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
       const int chunk = (lane & 3) ^ g8_swz64(r, S16);
       a_src[d] = (uint32_t)((int64_t)gm * p.lda) + chunk * 16;
     } else {
-      const int r = 8 * (8 * d + wave) + (lane >> 3);
+      const int r = 8 * (LOADERS * d + loader) + (lane >> 3);
       int gm = m0 + r;
       gm = gm < p.M ? gm : p.M - 1;
       const int chunk = (lane & 7) ^ (BF ? swz_pair(r) : g8_swz128(r, S16));
@@ -839,26 +851,28 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   uint32_t b_src[B_DMA];
 #pragma unroll
   for (int d = 0; d < B_DMA; ++d) {
-    const int r = BF ? 8 * (8 * d + wave) + (lane >> 3) : 16 * (8 * d + wave) + (lane >> 2);
+    const int r = MX ? 16 * (8 * d + wave) + (lane >> 2) : 8 * (LOADERS * d + loader) + (lane >> 3);
     int gn = n0 + r;
     gn = gn < p.N ? gn : p.N - 1;
-    const int chunk = BF ? (lane & 7) ^ swz_pair(r) : (lane & 3) ^ g8_swz64(r, S16);
+    const int chunk = MX ? (lane & 3) ^ g8_swz64(r, S16) : (lane & 7) ^ swz_pair(r);
     b_src[d] = (uint32_t)((int64_t)gn * p.ldb * (BF ? 2 : 1)) + chunk * 16;
   }
-  // BF: an operand's pair `pair` (clamped to the last one) into ring slot `slot`
-  const int last_pair = (KT >> 1) - 1;
-  auto dma_pair_a = [&](int pair, int slot) __attribute__((always_inline)) {
-    pair = pair < last_pair ? pair : last_pair;
+  // the activations' stage (BF: pair) `u` / the weights' pair, clamped to the
+  // last one, into ring slot `slot`.  A last half pair (W8, odd KT) reads on
+  // into the next row: in the operand or past its record count, and unused.
+  const int last_a = BF ? (KT >> 1) - 1 : KT - 1, last_b = ((KT + 1) >> 1) - 1;
+  auto dma_a = [&](int u, int slot) __attribute__((always_inline)) {
+    u = u < last_a ? u : last_a;
 #pragma unroll
     for (int d = 0; d < A_DMA; ++d)
-      buffer_dma16(p.A, a_records, a_src[d], pair * A_ROWB, lds + slot * A_BYTES + (8 * d + wave) * 1024);
+      buffer_dma16(p.A, a_records, a_src[d], u * A_ROWB, lds + slot * A_BYTES + (LOADERS * d + loader) * 1024);
   };
-  auto dma_pair_b = [&](int pair, int slot) __attribute__((always_inline)) {
-    pair = pair < last_pair ? pair : last_pair;
+  auto dma_b = [&](int u, int slot) __attribute__((always_inline)) {
+    u = u < last_b ? u : last_b;
 #pragma unroll
     for (int d = 0; d < B_DMA; ++d)
-      buffer_dma16(p.B, b_records, b_src[d], pair * B_ROWB,
-                   lds + B_REGION + slot * B_BYTES + (8 * d + wave) * 1024);
+      buffer_dma16(p.B, b_records, b_src[d], u * B_ROWB,
+                   lds + B_REGION + slot * B_BYTES + (LOADERS * d + loader) * 1024);
   };
   auto dma_stage = [&](int kt, int buf) __attribute__((always_inline)) {
     char* As = lds + buf * A_BYTES;
@@ -894,9 +908,8 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // The activation bases come as a low / high pair (stage buffers 0-1 / 1-2
   // of the 8-bit-code ring) so that the offsets fit the 16-bit immediate.
   const int r16 = lane & 15, q = lane >> 4;
-  // BF: chunk 4 s + q of the 128-byte row of a pair is the lane's fragment of
-  // its stage s; the weights' bases as a low / high pair too (slots 0 and 1-2).
-  const int w16 = B_REGION + (wn * WN + r16) * B_ROWB + ((q ^ g8_swz64(r16, true)) * 16);
+  // Pairs: chunk 4 s + q of a row is the lane's fragment of the pair's stage s;
+  // the weights' bases as a low / high pair too (slots 0 and 1-2).
   int x16_lo[2], x16_hi[2], w16_lo[2], w16_hi[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
@@ -935,8 +948,8 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   auto dma_scales = [&](int oct) {
     if constexpr (SCALED) {
       oct = oct < noct ? oct : noct - 1;  // past the end: re-read the last octet
-      if (grp == 0)
-        buffer_dma16(p.bscale, sc_records, sc_src, oct * 16, sc_lds + (oct & 1) * Cfg::SC_OCT + wave * 1024);
+      if (W8 || grp == 0)  // W8: called by group 1 only
+        buffer_dma16(p.bscale, sc_records, sc_src, oct * 16, sc_lds + (oct & 1) * Cfg::SC_OCT + (wave & 3) * 1024);
       else if (MX)
         buffer_dma16(p.ascale, asc_records, sc_src, oct * 16,
                      sc_lds + (2 + (oct & 1)) * Cfg::SC_OCT + (wave & 3) * 1024);
@@ -988,26 +1001,20 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
         for (int i = 0; i < TM; ++i)
           fa8[pp][i] = *reinterpret_cast<const u32x4*>(lds + a_mx[pp] + BUF * A_BYTES + i * 32 * A_ROWB);
       }
-    } else if constexpr (BF) {
-      // BUF = kt % STAGES: pair BUF / 2 in slots BUF / 2 % AP and % BP
-      constexpr int SA = BUF / 2 % AP, SB = BUF / 2 % BP, S = BUF & 1;
+    } else {
+      // BUF = kt % STAGES: the weights in slot BUF / 2 % BP, the activations
+      // in slot BUF / 2 % AP (BF) or BUF % AP
+      constexpr int SA = (BF ? BUF / 2 : BUF) % AP, SB = BUF / 2 % BP, S = BUF & 1;
       const int wb = SB == 0 ? w16_lo[S] : w16_hi[S] + (SB - 1) * B_BYTES;
-      const int xb = SA == 0 ? x16_lo[S] : x16_hi[S] + (SA - 1) * A_BYTES;
 #pragma unroll
       for (int jb = 0; jb < TN16; ++jb) w16f[jb] = *reinterpret_cast<const u32x4*>(lds + wb + jb * 16 * B_ROWB);
 #pragma unroll
-      for (int ib = 0; ib < TM16; ++ib) x16f[0][ib] = *reinterpret_cast<const bf16x8*>(lds + xb + ib * 16 * A_ROWB);
-    } else {
+      for (int s = 0; s < XS; ++s) {
+        const int h = BF ? S : s;
+        const int xb = SA == 0 ? x16_lo[h] : x16_hi[h] + (SA - 1) * A_BYTES;
 #pragma unroll
-      for (int jb = 0; jb < TN16; ++jb)
-        w16f[jb] = *reinterpret_cast<const u32x4*>(lds + w16 + BUF * B_BYTES + jb * 16 * B_ROWB);
-      const int* base = BUF == 0 ? x16_lo : x16_hi;
-      constexpr int rel = (BUF == 0 ? 0 : BUF - 1) * A_BYTES;
-#pragma unroll
-      for (int s = 0; s < XS; ++s)
-#pragma unroll
-        for (int ib = 0; ib < TM16; ++ib)
-          x16f[s][ib] = *reinterpret_cast<const bf16x8*>(lds + base[s] + rel + ib * 16 * A_ROWB);
+        for (int ib = 0; ib < TM16; ++ib) x16f[s][ib] = *reinterpret_cast<const bf16x8*>(lds + xb + ib * 16 * A_ROWB);
+      }
     }
   };
 
@@ -1122,17 +1129,29 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
     }
   };
 
-  // ---- prologue: scales of octet 0, stages 0 .. AHEAD-1 in flight, then one
-  // barrier for all waves
-  // BF: pairs in flight when pair b's loads must have landed -- those of the
-  // AP - 2 activation pairs and of the one weight pair after it
+  // ---- prologue: scales of octet 0 and all slots but one in flight, the first
+  // stage landed, then one barrier for all waves
+  // loads in flight when those of a pair (W8: a stage of the activations) must
+  // have landed: BF those of the AP - 2 activation pairs and of the one weight
+  // pair after it, W8 those of the AP - 2 stages or BP - 2 pairs after it
   constexpr int BF_FLIGHT = (AP - 2) * A_DMA + B_DMA;
+  constexpr int A_FLIGHT = (AP - 2) * A_DMA, B_FLIGHT = (BP - 2) * B_DMA;
   if constexpr (BF) {
-    dma_pair_a(0, 0);
-    dma_pair_b(0, 0);
-    if constexpr (AP == 3) dma_pair_a(1, 1);
-    dma_pair_b(1, 1);
+    dma_a(0, 0);
+    dma_b(0, 0);
+    if constexpr (AP == 3) dma_a(1, 1);
+    dma_b(1, 1);
     wait_vmcnt<BF_FLIGHT>();
+    barrier_nofence();
+  } else if constexpr (W8) {
+    if (grp == 0) {
+      static_for<0, AP - 1>([&](auto ic) { dma_a(decltype(ic)::value, decltype(ic)::value); });
+      wait_vmcnt<A_FLIGHT>();
+    } else {
+      dma_scales(0);
+      static_for<0, BP - 1>([&](auto ic) { dma_b(decltype(ic)::value, decltype(ic)::value); });
+      wait_vmcnt<B_FLIGHT>();
+    }
     barrier_nofence();
   } else {
     dma_scales(0);
@@ -1145,12 +1164,12 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
 
   // Clusters are whole stages.  Stage s is first read by group 0's memory
   // cluster of stage s (global half-stage 2s), so its data must be in LDS by
-  // the barrier before it.  The direct loads of stage s are issued in the
-  // memory clusters of stage s-AHEAD; each group waits for them in its last
+  // the barrier before it.  Direct loads go into the slot that stage s-1 left,
+  // in the memory cluster of stage s; each group waits for them in its last
   // cluster before that barrier -- group 0 at the end of its compute cluster
   // of stage s-1, group 1 at the end of its memory cluster of stage s-1 --
-  // leaving only the loads of the AHEAD-1 later stages in flight.  Past the last stage the
-  // direct loads re-read stage KT-1 into the buffer nobody reads any more,
+  // leaving only the loads of later stages in flight.  Past the last stage the
+  // direct loads re-read the last one into the buffer nobody reads any more,
   // so every stage issues the same loads and the waits are exact.  The scales
   // of octet o+1 go out (group 0) with stage 8o's loads.
   // BF: the memory cluster of a pair's first stage issues the activations'
@@ -1165,11 +1184,18 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
     constexpr bool PAIR_END = (BUF & 1) != 0;
     // memory cluster (MX: group 1 moves the activations' scale octets)
     if constexpr (BF) {
-      if (PAIR_END) dma_pair_b((kt >> 1) + BP - 1, (BUF / 2 + BP - 1) % BP);
-      else dma_pair_a((kt >> 1) + AP - 1, (BUF / 2 + AP - 1) % AP);
+      if (PAIR_END) dma_b((kt >> 1) + BP - 1, (BUF / 2 + BP - 1) % BP);
+      else dma_a((kt >> 1) + AP - 1, (BUF / 2 + AP - 1) % AP);
+    } else if constexpr (W8) {
+      if constexpr (GRP == 0) {
+        dma_a(kt + AP - 1, (BUF + AP - 1) % AP);
+      } else {
+        if (oct_start) dma_scales((kt >> 3) + 1);
+        if (!PAIR_END) dma_b((kt >> 1) + BP - 1, (BUF / 2 + BP - 1) % BP);
+      }
     } else {
-      if ((GRP == 0 || MX) && oct_start) dma_scales((kt >> 3) + 1);
-      dma_stage(kt + AHEAD < KT ? kt + AHEAD : KT - 1, (BUF + AHEAD) % STAGES);
+      if (oct_start) dma_scales((kt >> 3) + 1);
+      dma_stage(kt + 2 < KT ? kt + 2 : KT - 1, (BUF + 2) % STAGES);
     }
     if (live) read_stage(kt, bufc);
     wait_lgkmcnt0();
@@ -1177,7 +1203,9 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
     if (GRP == 1) {
       if constexpr (BF) {
         if (PAIR_END) wait_vmcnt<BF_FLIGHT>();
-      } else if (MX && oct_start) {
+      } else if constexpr (W8) {
+        if (PAIR_END) wait_vmcnt<B_FLIGHT>();
+      } else if (oct_start) {
         wait_vmcnt<VM_DMA + VM_SCALES>();
       } else {
         wait_vmcnt<VM_DMA>();
@@ -1191,6 +1219,8 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
     if (GRP == 0) {
       if constexpr (BF) {
         if (PAIR_END) wait_vmcnt<BF_FLIGHT>();
+      } else if constexpr (W8) {
+        wait_vmcnt<A_FLIGHT>();
       } else if (oct_start) {
         wait_vmcnt<VM_DMA + VM_SCALES>();
       } else {
