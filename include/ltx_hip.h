@@ -207,6 +207,32 @@ int ltx_gemv_f32_bf16w(const float* x, int64_t batch, int64_t K, const void* W,
                        void* stream);
 
 /*
+ * Up to 8 timestep MLPs (timestep_embedding.py:126-201), layer by layer in
+ * three launches: h1 = silu(w1 sinusoid(t[0] * multiplier) + b1), h2 = w2 h1 +
+ * b2 (the embedded timestep), out = w silu(h2) + b.  w1: bf16 (dim, 256); w2:
+ * (dim, dim); w: (num * dim, dim); t: one fp32 device scalar; biases fp32 or
+ * NULL; h1, h2 (dim) and out (num * dim) fp32 device rows.  dim <= 4096, a
+ * multiple of 8.  The same values as ltx_timestep_embedding_f32 and three
+ * ltx_gemv_f32_bf16w calls.
+ */
+typedef struct ltx_adaln_mlp {
+  const float* t;
+  const void* w1;
+  const float* b1;
+  const void* w2;
+  const float* b2;
+  const void* w;
+  const float* b;
+  float* h1;
+  float* h2;
+  float* out;
+  int64_t dim;
+  int64_t num;
+  float multiplier;
+} ltx_adaln_mlp;
+int ltx_adaln_mlps_f32(const ltx_adaln_mlp* mlps, int64_t count, void* stream);
+
+/*
  * out[b, i] = table[b, i] + vec[i] for b < nb, i < n (fp32): the AdaLN
  * modulation rows of every block, `scale_shift_table + timestep`
  * (transformer.py:286-342), computed for all blocks in one launch per step.

@@ -435,6 +435,16 @@ __global__ __launch_bounds__(256) void euler_kernel(const bf16* latent, const bf
   }
 }
 
+// column c of the sinusoidal embedding of timestep t (cosines, then sines);
+// exponent = (-ln(10000) * i) / half, each step rounded to fp32 as in the
+// reference's fp32 array arithmetic
+__device__ __forceinline__ float timestep_sinusoid(float t, int64_t c, int64_t half) {
+  const int64_t i = c < half ? c : c - half;
+  const float expo = __fdiv_rn(__fmul_rn(-9.210340371976184f, (float)i), (float)half);
+  const float arg = __fmul_rn(t, expf(expo));
+  return c < half ? cosf(arg) : sinf(arg);
+}
+
 __global__ void timestep_embedding_kernel(const float* values, int64_t count, float mult,
                                           float* out, int64_t dim) {
   const int64_t half = dim / 2;
@@ -445,13 +455,7 @@ __global__ void timestep_embedding_kernel(const float* values, int64_t count, fl
     out[idx] = 0.0f;
     return;
   }
-  const int64_t i = c < half ? c : c - half;
-  // exponent = (-ln(10000) * i) / half, each step rounded to fp32 as in the
-  // reference's fp32 array arithmetic.
-  const float expo = __fdiv_rn(__fmul_rn(-9.210340371976184f, (float)i), (float)half);
-  const float t = __fmul_rn(values[b], mult);
-  const float arg = __fmul_rn(t, expf(expo));
-  out[idx] = c < half ? cosf(arg) : sinf(arg);
+  out[idx] = timestep_sinusoid(__fmul_rn(values[b], mult), c, half);
 }
 
 // GEMV: each wave computes kGemvRowsPerWave outputs for every batch entry;
@@ -517,6 +521,86 @@ __global__ __launch_bounds__(256) void gemv_kernel(const float* __restrict__ x, 
       }
     }
   }
+}
+
+// One layer of several timestep MLPs in one launch (ltx_adaln_mlps_f32):
+// workgroups [first_block, next first_block) take one MLP's rows, rows_per_block
+// each, so that every workgroup streams about the same bytes.  Bound by the
+// weight bytes (16 D x D rows of bf16 per modality): a wave has two rows'
+// loads in flight, the first issued before x is staged, and a row's next one
+// goes out as soon as it is summed.  The sums are those of gemv_kernel, in the
+// same order.  The eight MLPs of a step (D = 4096 and 2048, 850 MB) take 9 +
+// 50 + 161 us (the last layer at 4.2 TB/s), against 456 us as 32 dependent
+// launches of one layer each (1.7-3.3 TB/s).
+constexpr int kMaxMlps = 8;
+constexpr int kMlpSinusoid = 256;
+constexpr int kMlpBlocks = 1536;  // about two rounds of the three workgroups a CU holds
+struct MlpLayer {
+  const float* x;  // layer 0: the timestep
+  const bf16* W;
+  const float* bias;
+  float* y;
+  int N, K, rows_per_block, first_block;
+  float mult;
+};
+struct MlpGroup {
+  MlpLayer m[kMaxMlps];
+  int count;
+};
+
+template <int LAYER, int KIT>
+__device__ __forceinline__ void mlp_rows(const MlpLayer& m, float* xs) {
+  const int K = m.K, lane = threadIdx.x & (kWave - 1);
+  const int b0 = ((int)blockIdx.x - m.first_block) * m.rows_per_block;
+  const int end = b0 + m.rows_per_block < m.N ? b0 + m.rows_per_block : m.N;
+  bf16x8 wv[kGemvRowsPerWave][KIT];
+  auto load = [&](int rr, int n) {
+    n = n < m.N ? n : m.N - 1;
+#pragma unroll
+    for (int j = 0; j < KIT; ++j) {
+      const int k0 = lane * 8 + j * kWave * 8;
+      if (k0 < K) wv[rr][j] = *reinterpret_cast<const bf16x8*>(m.W + (int64_t)n * K + k0);
+    }
+  };
+  int n0 = b0 + (threadIdx.x >> 6) * kGemvRowsPerWave;
+#pragma unroll
+  for (int rr = 0; rr < kGemvRowsPerWave; ++rr) load(rr, n0 + rr);
+  const float t = LAYER == 0 ? __fmul_rn(m.x[0], m.mult) : 0.0f;
+  for (int i = threadIdx.x; i < K; i += 256)
+    xs[i] = LAYER == 0 ? timestep_sinusoid(t, i, K / 2) : (LAYER == 2 ? silu(m.x[i]) : m.x[i]);
+  __syncthreads();
+  constexpr int STEP = 4 * kGemvRowsPerWave;
+  for (; n0 < end; n0 += STEP) {
+#pragma unroll
+    for (int rr = 0; rr < kGemvRowsPerWave; ++rr) {
+      float acc = 0.0f;
+#pragma unroll
+      for (int j = 0; j < KIT; ++j) {
+        const int k0 = lane * 8 + j * kWave * 8;
+        if (k0 < K) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc = fmaf((float)wv[rr][j][i], xs[k0 + i], acc);
+        }
+      }
+      if (n0 + STEP < end) load(rr, n0 + STEP + rr);
+      float v = wave_sum(acc);
+      if (lane == 0 && n0 + rr < end) {
+        if (m.bias) v += m.bias[n0 + rr];
+        m.y[n0 + rr] = LAYER == 0 ? silu(v) : v;
+      }
+    }
+  }
+}
+
+// LAYER 0: sinusoid(t) -> linear_1 -> SiLU; 1: linear_2; 2: SiLU -> linear
+template <int LAYER>
+__global__ __launch_bounds__(256) void mlp_layer_kernel(MlpGroup g) {
+  __shared__ __attribute__((aligned(16))) float xs[LAYER == 0 ? kMlpSinusoid : kGemvMaxK];
+  int i = 0;
+  while (i + 1 < g.count && (int)blockIdx.x >= g.m[i + 1].first_block) ++i;
+  if constexpr (LAYER == 0) mlp_rows<0, 1>(g.m[i], xs);
+  else if (g.m[i].K <= 2048) mlp_rows<LAYER, 4>(g.m[i], xs);
+  else mlp_rows<LAYER, 8>(g.m[i], xs);
 }
 
 // out[b, i] = table[b, i] + vec[i]  (per-block AdaLN modulation rows)
@@ -825,6 +909,50 @@ extern "C" int ltx_gemv_f32_bf16w(const float* x, int64_t batch, int64_t K, cons
     gemv_kernel<4><<<(int)blocks, 256, lds, s>>>(x, (int)batch, (int)K, w, bias, y, N, flags);
   else
     gemv_kernel<8><<<(int)blocks, 256, lds, s>>>(x, (int)batch, (int)K, w, bias, y, N, flags);
+  return ltx_launch_status();
+}
+
+extern "C" int ltx_adaln_mlps_f32(const ltx_adaln_mlp* mlps, int64_t count, void* stream) {
+  if (count < 0 || (count > 0 && !mlps)) return LTX_ERR_INVALID_ARG;
+  if (count > kMaxMlps) return LTX_ERR_UNSUPPORTED;
+  for (int64_t i = 0; i < count; ++i) {
+    const ltx_adaln_mlp& m = mlps[i];
+    if (!m.t || !m.w1 || !m.w2 || !m.w || !m.h1 || !m.h2 || !m.out || m.dim <= 0 || m.num <= 0)
+      return LTX_ERR_INVALID_ARG;
+    if (m.dim > kGemvMaxK || m.dim % 8 || m.num > INT32_MAX / (2 * m.dim)) return LTX_ERR_UNSUPPORTED;
+    if (!aligned16(m.w1) || !aligned16(m.w2) || !aligned16(m.w)) return LTX_ERR_ALIGNMENT;
+  }
+  if (count == 0) return LTX_OK;
+  hipStream_t s = (hipStream_t)stream;
+  for (int layer = 0; layer < 3; ++layer) {
+    MlpGroup g{};
+    g.count = (int)count;
+    int64_t bytes = 0;
+    for (int64_t i = 0; i < count; ++i) {
+      const ltx_adaln_mlp& m = mlps[i];
+      MlpLayer& l = g.m[i];
+      l.x = layer == 0 ? m.t : (layer == 1 ? m.h1 : m.h2);
+      l.W = (const bf16*)(layer == 0 ? m.w1 : (layer == 1 ? m.w2 : m.w));
+      l.bias = layer == 0 ? m.b1 : (layer == 1 ? m.b2 : m.b);
+      l.y = layer == 0 ? m.h1 : (layer == 1 ? m.h2 : m.out);
+      l.K = layer == 0 ? kMlpSinusoid : (int)m.dim;
+      l.N = (int)(layer == 2 ? m.num * m.dim : m.dim);
+      l.mult = m.multiplier;
+      bytes += (int64_t)l.N * l.K;
+    }
+    constexpr int STEP = 4 * kGemvRowsPerWave;  // rows of one pass of a workgroup
+    int blocks = 0;
+    for (int64_t i = 0; i < count; ++i) {
+      MlpLayer& l = g.m[i];
+      const int64_t passes = (bytes / kMlpBlocks + (int64_t)STEP * l.K - 1) / ((int64_t)STEP * l.K);
+      l.rows_per_block = (int)((passes < 1 ? 1 : passes) * STEP);
+      l.first_block = blocks;
+      blocks += (l.N + l.rows_per_block - 1) / l.rows_per_block;
+    }
+    if (layer == 0) mlp_layer_kernel<0><<<blocks, 256, 0, s>>>(g);
+    else if (layer == 1) mlp_layer_kernel<1><<<blocks, 256, 0, s>>>(g);
+    else mlp_layer_kernel<2><<<blocks, 256, 0, s>>>(g);
+  }
   return ltx_launch_status();
 }
 

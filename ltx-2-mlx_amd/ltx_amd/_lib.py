@@ -36,6 +36,7 @@ SIGNATURES: dict[str, list] = {
     "ltx_output_norm_modulate_bf16": [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp],
     "ltx_euler_x0_step_bf16": [_vp, _vp, _f32, _f32, _vp, _i64, _vp],
     "ltx_timestep_embedding_f32": [_vp, _i64, _f32, _vp, _i64, _vp],
+    "ltx_adaln_mlps_f32": [_vp, _i64, _vp],
     "ltx_gemv_f32_bf16w": [_vp, _i64, _i64, _vp, _vp, _vp, _i64, _int, _vp],
     "ltx_gemm_bf16": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64, _vp, _i64, _vp],
     "ltx_gemm_w8a16_bf16": [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64, _vp,

@@ -27,7 +27,7 @@ from ... import _lib
 from ...kernels import gemm
 from ...loader.weights import build_block, linear_weight
 from .rope import AUDIO_MAX_POS, VIDEO_MAX_POS, rope_tables
-from .timestep_embedding import SINUSOID_DIM, AdaLayerNormSingle
+from .timestep_embedding import AdaLayerNormSingle, run_mlps
 from .transformer import ADA_ROWS, BasicAVTransformerBlock, TransformerArgs, TransformerConfig
 
 AUDIO_HEADS = 32
@@ -283,7 +283,12 @@ class LTXModel:
 
     def _timestep_rows(self, sigma_dev: torch.Tensor, cross_sigma_dev: torch.Tensor, video: bool,
                        prompt_sigma_dev: torch.Tensor | None = None) -> None:
-        """Fill the (16, D) timestep rows of one modality (model.py:160-187,
+        """Run :meth:`_timestep_jobs` of one modality."""
+        run_mlps(self._timestep_jobs(sigma_dev, cross_sigma_dev, video, prompt_sigma_dev))
+
+    def _timestep_jobs(self, sigma_dev: torch.Tensor, cross_sigma_dev: torch.Tensor, video: bool,
+                       prompt_sigma_dev: torch.Tensor | None = None) -> list:
+        """The timestep MLPs (``run_mlps`` jobs) that fill the (16, D) timestep rows of one modality (model.py:160-187,
         :305-314, :418-497) and its embedded timestep: the AdaLN rows 0-8 and
         the cross scale / shift rows 11-14 from the modality's timestep, the
         prompt rows 9-10 from its sigma (``prompt_sigma_dev``, default the
@@ -294,13 +299,14 @@ class LTXModel:
         ts = self.timestep_scale_multiplier
         mlps = self._mlps(video)
         flat = temb.view(-1)
-        mlps[0](sigma_dev, ts, flat[: 9 * d], embedded=emb)
-        mlps[1](sigma_dev if prompt_sigma_dev is None else prompt_sigma_dev, ts, flat[9 * d: 11 * d])
+        jobs = [(mlps[0], sigma_dev, ts, flat[: 9 * d], emb),
+                (mlps[1], sigma_dev if prompt_sigma_dev is None else prompt_sigma_dev, ts, flat[9 * d: 11 * d], None)]
         if self.audio_config is not None:
-            mlps[2](sigma_dev, ts, flat[11 * d: 15 * d])
-            mlps[3](cross_sigma_dev, self.av_ca_timestep_scale_multiplier, flat[15 * d: 16 * d])
+            jobs += [(mlps[2], sigma_dev, ts, flat[11 * d: 15 * d], None),
+                     (mlps[3], cross_sigma_dev, self.av_ca_timestep_scale_multiplier, flat[15 * d: 16 * d], None)]
         else:
             flat[11 * d:].zero_()
+        return jobs
 
     def _token_group_rows(self, groups: TokenTimesteps) -> tuple[torch.Tensor, torch.Tensor]:
         """Per-token video timesteps as row groups: for each distinct value
@@ -392,7 +398,10 @@ class LTXModel:
 
         # preprocess
         vx = project(video_latent, self.patchify_proj)
-        self._timestep_rows(vt, as_, video=True, prompt_sigma_dev=vs)
+        jobs = self._timestep_jobs(vt, as_, video=True, prompt_sigma_dev=vs)
+        if run_audio:
+            jobs += self._timestep_jobs(at, vs, video=False, prompt_sigma_dev=as_)
+        run_mlps(jobs)
         stream = _lib.stream_of(vx)
         _lib.call("ltx_broadcast_add_f32", self.video_tables.data_ptr(), self._temb_v.data_ptr(),
                   self._ada_v.data_ptr(), self.num_layers, ADA_ROWS * self.video_dim, stream)
@@ -401,7 +410,6 @@ class LTXModel:
         audio = None
         if run_audio:
             ax = project(audio_latent, self.audio_patchify_proj)
-            self._timestep_rows(at, vs, video=False, prompt_sigma_dev=as_)
             _lib.call("ltx_broadcast_add_f32", self.audio_tables.data_ptr(), self._temb_a.data_ptr(),
                       self._ada_a.data_ptr(), self.num_layers, ADA_ROWS * self.audio_dim, stream)
             audio = TransformerArgs(x=ax, context=audio_context, timesteps=self._temb_a[:9],

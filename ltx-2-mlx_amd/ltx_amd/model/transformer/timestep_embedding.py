@@ -3,17 +3,45 @@
 ``AdaLayerNormSingle(t) -> (emb (N*D), embedded_timestep (D))`` with
 sinusoid(256, flip_sin_to_cos, shift 0) -> linear_1 -> SiLU -> linear_2
 (= embedded_timestep) -> SiLU -> linear(D -> N*D) (:126-201).  The three
-layers run as fp32-activation / bf16-weight GEMV kernels; the final layer
-writes straight into a slice of the caller's modulation-row buffer.
+layers run as fp32-activation / bf16-weight GEMV kernels, each layer of all the
+MLPs of a step in one launch (:func:`run_mlps`); the final layer writes
+straight into a slice of the caller's modulation-row buffer.
 """
 
 from __future__ import annotations
+
+import ctypes
 
 import torch
 
 from ... import _lib
 
 SINUSOID_DIM = 256
+MAX_MLPS = 8  # per ltx_adaln_mlps_f32 call
+
+
+class _MlpArgs(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("t", "w1", "b1", "w2", "b2", "w", "b", "h1", "h2", "out")] + [
+        ("dim", ctypes.c_int64), ("num", ctypes.c_int64), ("multiplier", ctypes.c_float)]
+
+
+def run_mlps(jobs: list, scratch: list | None = None) -> None:
+    """Run independent timestep MLPs together: each job is (mlp, t_value,
+    multiplier, out, embedded or None), as for ``AdaLayerNormSingle.__call__``;
+    ``scratch``: (hidden, embedded) fp32 rows per job (default: allocated)."""
+    for i in range(0, len(jobs), MAX_MLPS):
+        part = jobs[i:i + MAX_MLPS]
+        dev = part[0][3].device
+        rows = (torch.empty((len(part), 2, max(j[0].dim for j in part)), device=dev) if scratch is None
+                else scratch[i:i + MAX_MLPS])
+        args = (_MlpArgs * len(part))()
+        for a, h, (m, t, mult, out, embedded) in zip(args, rows, part):
+            h2 = h[1] if embedded is None else embedded
+            a.t, a.w1, a.b1, a.w2, a.b2 = t.data_ptr(), m.w1.data_ptr(), m.b1.data_ptr(), m.w2.data_ptr(), m.b2.data_ptr()
+            a.w, a.b, a.h1, a.h2, a.out = m.w.data_ptr(), m.b.data_ptr(), h[0].data_ptr(), h2.data_ptr(), out.data_ptr()
+            a.dim, a.num, a.multiplier = m.dim, m.num_embeddings, float(mult)
+        _lib.call("ltx_adaln_mlps_f32", ctypes.addressof(args), len(part), _lib.stream_of(part[0][3]),
+                  detail=f"{len(part)} timestep MLPs")
 
 
 class AdaLayerNormSingle:
@@ -39,21 +67,4 @@ class AdaLayerNormSingle:
                  embedded: torch.Tensor | None = None, scratch: tuple | None = None) -> None:
         """t_value: fp32 device scalar (1,); writes emb (N*D) into ``out`` and,
         if given, embedded_timestep (D) into ``embedded``."""
-        dev = out.device
-        stream = _lib.stream_of(out)
-        if scratch is None:
-            sin = torch.empty(SINUSOID_DIM, device=dev)
-            h1 = torch.empty(self.dim, device=dev)
-            h2 = torch.empty(self.dim, device=dev) if embedded is None else embedded
-        else:
-            sin, h1, h2 = scratch
-            if embedded is not None:
-                h2 = embedded
-        _lib.call("ltx_timestep_embedding_f32", t_value.data_ptr(), 1, float(multiplier), sin.data_ptr(),
-                  SINUSOID_DIM, stream)
-        _lib.call("ltx_gemv_f32_bf16w", sin.data_ptr(), 1, SINUSOID_DIM, self.w1.data_ptr(), self.b1.data_ptr(),
-                  h1.data_ptr(), self.dim, _lib.GEMV_SILU_OUTPUT, stream)
-        _lib.call("ltx_gemv_f32_bf16w", h1.data_ptr(), 1, self.dim, self.w2.data_ptr(), self.b2.data_ptr(),
-                  h2.data_ptr(), self.dim, 0, stream)
-        _lib.call("ltx_gemv_f32_bf16w", h2.data_ptr(), 1, self.dim, self.w.data_ptr(), self.b.data_ptr(),
-                  out.data_ptr(), self.num_embeddings * self.dim, _lib.GEMV_SILU_INPUT, stream)
+        run_mlps([(self, t_value, multiplier, out, embedded)], None if scratch is None else [scratch[1:]])
