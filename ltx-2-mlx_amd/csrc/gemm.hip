@@ -858,8 +858,9 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
     b_src[d] = (uint32_t)((int64_t)gn * p.ldb * (BF ? 2 : 1)) + chunk * 16;
   }
   // the activations' stage (BF: pair) `u` / the weights' pair, clamped to the
-  // last one, into ring slot `slot`.  A last half pair (W8, odd KT) reads on
-  // into the next row: in the operand or past its record count, and unused.
+  // last one, into ring slot `slot`.  In a last half pair (int8, odd KT) the
+  // lanes of the missing stage read the other one's bytes again, so that no
+  // load leaves its row (the record count does not bound the scalar offset).
   const int last_a = BF ? (KT >> 1) - 1 : KT - 1, last_b = ((KT + 1) >> 1) - 1;
   auto dma_a = [&](int u, int slot) __attribute__((always_inline)) {
     u = u < last_a ? u : last_a;
@@ -869,6 +870,16 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   };
   auto dma_b = [&](int u, int slot) __attribute__((always_inline)) {
     u = u < last_b ? u : last_b;
+    if constexpr (BKIND == B_INT8) {
+      if (u == last_b && (KT & 1)) {
+        const uint32_t back = (((lane & 7) ^ swz_pair(lane >> 3)) & 4) * 16;
+#pragma unroll
+        for (int d = 0; d < B_DMA; ++d)
+          buffer_dma16(p.B, b_records, b_src[d] - back, u * B_ROWB,
+                       lds + B_REGION + slot * B_BYTES + (LOADERS * d + loader) * 1024);
+        return;
+      }
+    }
 #pragma unroll
     for (int d = 0; d < B_DMA; ++d)
       buffer_dma16(p.B, b_records, b_src[d], u * B_ROWB,
