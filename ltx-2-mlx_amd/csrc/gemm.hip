@@ -1519,6 +1519,13 @@ static double kg_time(int bkind, int64_t M, int64_t N, int64_t K, int bm, int64_
   return t;
 }
 
+// The same for 128x128 tiles of gemm_kernel, at most one workgroup per CU (0.6
+// us per 64 k in every format: bf16 77 x 188160 -> 2048 in 4 splits 450 us).
+static double tile128_time(int64_t M, int64_t N, int64_t K, int64_t splits) {
+  const double t = (double)(K / 64) / (double)splits * 0.6 + 4.0;
+  return splits > 1 ? t + 3.5 + (double)(M * N * splits) * 8.0 / 3.5e6 : t;
+}
+
 // The tile height that the model finds fastest for a split count.
 static int kg_rows(int bkind, int64_t M, int64_t N, int64_t K, int64_t splits, double* us) {
   int best = 64;
@@ -1951,29 +1958,42 @@ extern "C" int ltx_gemm_mx_gelu_mxfp8(const uint8_t* A, int64_t lda, const uint8
 }
 
 // Split-K factor that the library would choose for a product (wformat 0:
-// bf16, 1: int8, 2: MXFP8): the power of two that models fastest while the
-// splits still fit one round of the 256 CUs, taken over fewer splits only
-// when it models >= 15 % faster (a second launch and a workspace).
+// bf16, 1: int8, 2: MXFP8): the count that models fastest, of those that leave
+// whole units of K per split (at least 256 k: bf16 8 x 1024 -> 2048 9.9 us in 8
+// splits of one unit, 7.3 in one pass) and fit one round of the 256 CUs.  All
+// divisors count, not the powers of two alone: bf16 77 x 188160 -> 2048 161 us
+// in 14 splits, 567 in 2 (a quarter of that depth is no whole number of units);
+// int8 68 x 8448 -> 248 34 us in 2, 16 in 11.  A split must
+// model 15 % faster than the single pass (it adds a launch and a workspace)
+// and 10 % faster than a smaller count: over 213 measured products of 26-1024
+// rows the choice is on average 1.1 % from the fastest count (15 % at every
+// step: 1.8 %, 384 x 16384 -> 4096 bf16 2 splits 88 us for 4 splits 69).
+// Depths that the mid-size kernel does not take (K / splits no multiple of its
+// unit) split on 128x128 tiles, few rows only, up to 80 workgroups: MXFP8 68 x
+// 3840 -> 4096 27 us in 2 splits against 40 in one pass, 68 x 1280 -> 2048 12.4
+// in 5 against 16.5.
 extern "C" int ltx_gemm_auto_splits(int64_t M, int64_t N, int64_t K, int wformat) {
   if (M <= 0 || N <= 0 || K <= 0 || wformat < 0 || wformat > 2 || M > INT32_MAX / 2 || N > INT32_MAX / 2 ||
       K > INT32_MAX / 2)
     return 1;
+  if (((M + 255) / 256) * ((N + 255) / 256) >= 100) return 1;
   const int64_t ld_scale = wformat == B_MXFP8 ? K / 32 : 0;
-  if (((M + 255) / 256) * ((N + 255) / 256) >= 100 || !kg_ok(wformat, M, N, K, K, K, ld_scale)) return 1;
-  // A split must model 15 % faster than the single pass (it adds a launch) and
-  // 10 % faster than a smaller split: over 213 measured products of 26-1024
-  // rows the choice is on average 1.1 % from the fastest count (15 % at every
-  // doubling: 1.8 %, 384 x 16384 -> 4096 bf16 2 splits 88 us for 4 splits 69,
-  // 121 x 4096 -> 4096 24.0 for 18.9).
-  double single, best;
-  kg_rows(wformat, M, N, K, 1, &single);
-  best = single;
+  const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128), unit128 = wformat == B_MXFP8 ? 128 : 64;
+  double single = tile128_time(M, N, K, 1);
+  if (kg_ok(wformat, M, N, K, K, K, ld_scale)) kg_rows(wformat, M, N, K, 1, &single);
+  double best = single;
   int splits = 1;
-  for (int s = 2; s <= 16; s *= 2) {
-    if (K % s || !kg_ok(wformat, M, N, K / s, K, K, ld_scale)) break;
+  for (int s = 2; s <= 16; ++s) {
+    if (K % s || K / s < 256) continue;
     double us;
-    const int bm = kg_rows(wformat, M, N, K, s, &us);
-    if (((M + bm - 1) / bm) * ((N + 127) / 128) * s > 256) continue;
+    if (kg_ok(wformat, M, N, K / s, K, K, ld_scale)) {
+      const int bm = kg_rows(wformat, M, N, K, s, &us);
+      if (((M + bm - 1) / bm) * ((N + 127) / 128) * s > 256) continue;
+    } else if (M <= 256 && K / s % unit128 == 0 && tiles128 * s <= 80) {
+      us = tile128_time(M, N, K, s);
+    } else {
+      continue;
+    }
     if (us < 0.85 * single && us < 0.9 * best) {
       best = us;
       splits = s;

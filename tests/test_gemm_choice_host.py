@@ -1,0 +1,43 @@
+"""The library's automatic GEMM choices (host code of csrc/gemm.hip), without a
+GPU: split counts for every depth the entry points take."""
+
+from __future__ import annotations
+
+import pytest
+
+KINDS = ["bf16", "int8", "mxfp8"]
+
+
+@pytest.fixture(scope="module")
+def gemm():
+    from ltx_amd import _lib
+    from ltx_amd.kernels import gemm
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libltx_hip.so not built")
+    return gemm
+
+
+@pytest.mark.parametrize("m,n,k,kind,least", [
+    (77, 2048, 188160, "bf16", 5),   # 188160 / 4 is no multiple of 128
+    (26, 2048, 188160, "bf16", 5),
+    (59, 248, 8448, "int8", 3),      # 8448 = 128 * 66
+    (1, 648, 10368, "int8", 3),      # 10368 = 128 * 81
+    (68, 4096, 3840, "mxfp8", 2),    # no multiple of 512: 128x128 tiles
+    (68, 2048, 1280, "mxfp8", 2),
+    (2, 448, 20224, "mxfp8", 2),
+    (3, 3480, 4736, "int8", 2),      # 37 units, split in halves of 64 k
+])
+def test_few_row_products_split_at_any_depth(gemm, m, n, k, kind, least):
+    assert gemm.auto_splits(m, n, k, kind) >= least
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_split_counts_are_counts_the_entry_points_take(gemm, kind):
+    unit = 128 if kind == "mxfp8" else 64
+    for m in (1, 26, 77, 256, 300, 1024):
+        for n in (8, 264, 2048, 4128):
+            for k in range(unit, 20000, 11 * unit):
+                s = gemm.auto_splits(m, n, k, kind)
+                assert 1 <= s <= 64 and k % (unit * s) == 0
+                assert s == 1 or k // s >= 256
