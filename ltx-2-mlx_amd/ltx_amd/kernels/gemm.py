@@ -147,11 +147,29 @@ def dequantize(weight: LinearWeight) -> torch.Tensor:
 _WFORMAT = {"bf16": 0, "int8": 1, "mxfp8": 2}
 
 
+# Block budget of a split-K launch on explicit 128x128 tiles (tiles x splits).
+SPLITK_MAX_BLOCKS = 80
+
+
 @functools.lru_cache(maxsize=4096)
-def auto_splits(m: int, n: int, k: int, kind: str) -> int:
+def auto_splits(m: int, n: int, k: int, kind: str, max_blocks: int | None = None) -> int:
     """Split-K factor of a product whose output tiles leave CUs idle, from the
-    library's cost model (ltx_gemm_auto_splits); 1 when one pass is as fast."""
-    return _lib.lib().ltx_gemm_auto_splits(m, n, k, _WFORMAT.get(kind, -1))
+    library's cost model (ltx_gemm_auto_splits); 1 when one pass is as fast.
+    With ``max_blocks``, the rule for few rows on 128x128 tiles instead: the
+    largest power of two that keeps at most that many blocks and at least 256
+    of K per split."""
+    if max_blocks is None:
+        return _lib.lib().ltx_gemm_auto_splits(m, n, k, _WFORMAT.get(kind, -1))
+    if m > 256 or k < 1024:
+        return 1
+    tiles = ((m + 127) // 128) * ((n + 127) // 128)
+    if tiles >= 160:
+        return 1
+    unit = 128 if kind == "mxfp8" else 64
+    s = 1
+    while tiles * s * 2 <= max_blocks and k % (unit * s * 2) == 0 and k // (s * 2) >= 256:
+        s *= 2
+    return s
 
 
 # Few-row products (at most ROWS_MAX_M rows: the 68 / 121-token audio stream)
@@ -443,7 +461,8 @@ def linear(x: torch.Tensor, weight: LinearWeight, *, epilogue: int = EPI_BIAS,
     With ``EPI_BIAS``, columns ``n >= sigmoid_from`` get the 2*sigmoid head
     gate instead (fused gate-logit columns of a Q/QKV projection).
     ``splits``: split-K factor (None: ``auto_splits`` with the automatic tile
-    choice, 1: single pass); the split form sums fp32 partials from a workspace.
+    choice and for the 128x128 tiles, 1: single pass); the split form sums fp32
+    partials from a workspace.
     With ``ROWS_KERNEL`` set, few-row products with ``splits=None`` and the
     automatic tile choice run on :func:`linear_rows`.
     """
@@ -496,7 +515,8 @@ def linear(x: torch.Tensor, weight: LinearWeight, *, epilogue: int = EPI_BIAS,
     hook = LAUNCH_HOOK
     info = (weight.kind, m, n, k, epilogue) if hook is not None else None
     if splits is None:
-        splits = auto_splits(m, n, k, weight.kind) if tile == TILE_AUTO else 1
+        splits = (auto_splits(m, n, k, weight.kind) if tile == TILE_AUTO else
+                  auto_splits(m, n, k, weight.kind, SPLITK_MAX_BLOCKS) if tile == TILE_128 else 1)
     if hook is not None:
         hook("pre", info)
     if splits == 1 and _mx_eligible(m, n, k, weight, tile):

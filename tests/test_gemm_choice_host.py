@@ -1,9 +1,11 @@
 """The library's automatic GEMM choices (host code of csrc/gemm.hip), without a
-GPU: split counts for every depth the entry points take."""
+GPU: split counts for every depth the entry points take, and the entry that
+linear() calls."""
 
 from __future__ import annotations
 
 import pytest
+import torch
 
 KINDS = ["bf16", "int8", "mxfp8"]
 
@@ -41,3 +43,18 @@ def test_split_counts_are_counts_the_entry_points_take(gemm, kind):
                 s = gemm.auto_splits(m, n, k, kind)
                 assert 1 <= s <= 64 and k % (unit * s) == 0
                 assert s == 1 or k // s >= 256
+
+
+@pytest.mark.parametrize("m,n,k,splits", [(68, 2048, 8192, 4), (121, 2048, 2048, 4), (256, 4096, 4096, 1),
+                                          (257, 2048, 8192, 1), (68, 2048, 512, 1)])
+def test_explicit_128_tiles_still_split(gemm, monkeypatch, m, n, k, splits):
+    """linear() on explicit 128x128 tiles splits few-row products by the
+    block budget of those tiles."""
+    calls = []
+    monkeypatch.setattr(gemm._lib, "call", lambda name, *args, detail="": calls.append((name, args)))
+    monkeypatch.setattr(gemm._lib, "stream_of", lambda t: 0)
+    weight = gemm.LinearWeight(kind="bf16", w=torch.empty((n, k), dtype=torch.bfloat16))
+    gemm.linear(torch.empty((m, k), dtype=torch.bfloat16), weight, tile=gemm.TILE_128)
+    (name, args), = calls
+    assert name == ("ltx_gemm_splitk_bf16" if splits > 1 else "ltx_gemm_bf16")
+    assert splits == 1 or args[15] == splits
