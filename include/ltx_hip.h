@@ -366,6 +366,10 @@ int64_t ltx_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int64_t splits);
 /* The split count the library would choose (1: one pass) for a product of
  * weight format `wformat` (0 bf16, 1 int8, 2 MXFP8). */
 int ltx_gemm_auto_splits(int64_t M, int64_t N, int64_t K, int wformat);
+/* The tile height (64, 128 or 192 rows) of an automatic launch of `splits` K
+ * ranges (1: the plain entry points) on the mid-size kernel, 0 where it takes
+ * another kernel. */
+int ltx_gemm_auto_rows(int64_t M, int64_t N, int64_t K, int wformat, int splits);
 int ltx_gemm_splitk_bf16(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias,
                          void* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int epilogue,
                          const void* residual, int64_t ldr, const float* gate, int64_t sigmoid_from,

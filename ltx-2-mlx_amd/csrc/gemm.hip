@@ -1548,13 +1548,20 @@ static int kg_rows(int bkind, int64_t M, int64_t N, int64_t K, int64_t splits, d
 // kernel against that one, K = 4096: 1728 x 4096 bf16 78 / 76, MXFP8 61 / 73;
 // 2048 x 4096 86 / 76, 67 / 77; 2304 x 4096 81 / 75, 81 / 75; 384 x 16384
 // 55 / 71, 51 / 76; 512 x 16384 93 / 77, 74 / 76; 700 x 12320 90 / 79, 86 / 77.
-static bool kg_auto(int bkind, const GemmArgs& p) {
-  const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
-  if (big >= 160 || !kg_ok(bkind, p.M, p.N, p.K, p.lda, p.ldb, p.ld_scale)) return false;
+// Shallow products of more than one round of 64-row tiles keep the older
+// kernels: with one to three units the loop is over before the ring has filled,
+// and two 128x128 workgroups per CU hide one's first loads behind the other's
+// epilogue (1296 x 128 -> 2048 bf16 7.3 / 6.6, 700 x 256 -> 4096 8.1 / 7.5, int8
+// 700 x 128 -> 4096 7.7 / 6.8, 1296 x 384 -> 2048 10.1 / 9.7; one round, 700 x
+// 128 -> 2048 bf16 5.8 / 6.1).
+static bool kg_auto(int bkind, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ld_scale) {
+  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
+  if (big >= 160 || !kg_ok(bkind, M, N, K, lda, ldb, ld_scale)) return false;
+  if (K <= (bkind == B_INT8 ? 384 : 256) && ((M + 63) / 64) * ((N + 127) / 128) > 256) return false;
   if (big < 100) return true;
   double us;
-  kg_rows(bkind, p.M, p.N, p.K, 1, &us);
-  return us < 4.0 + (p.K / 128) * (bkind == B_INT8 ? 2.4 : 2.1);
+  kg_rows(bkind, M, N, K, 1, &us);
+  return us < 4.0 + (K / 128) * (bkind == B_INT8 ? 2.4 : 2.1);
 }
 
 // Tile shapes (all K step 64): 256x256 and 128x128 with the register-staged
@@ -1564,7 +1571,7 @@ static bool kg_auto(int bkind, const GemmArgs& p) {
 template <int BKIND, int EPI>
 static int launch_epi_w(const GemmArgs& p, int tile, hipStream_t s) {
   const bool auto_tile = tile == 0;
-  if (auto_tile && kg_auto(BKIND, p)) {
+  if (auto_tile && kg_auto(BKIND, p.M, p.N, p.K, p.lda, p.ldb, p.ld_scale)) {
     kg_launch(BKIND, p, EPI, kg_rows(BKIND, p.M, p.N, p.K, 1, nullptr), 1, s);
     return LTX_OK;
   }
@@ -2000,6 +2007,18 @@ extern "C" int ltx_gemm_auto_splits(int64_t M, int64_t N, int64_t K, int wformat
     }
   }
   return splits;
+}
+
+// Tile height (64, 128, 192) of an automatic launch of `splits` K ranges on the
+// mid-size kernel, 0 where it takes another kernel; dense operands.
+extern "C" int ltx_gemm_auto_rows(int64_t M, int64_t N, int64_t K, int wformat, int splits) {
+  if (M <= 0 || N <= 0 || K <= 0 || wformat < 0 || wformat > 2 || M > INT32_MAX / 2 || N > INT32_MAX / 2 ||
+      K > INT32_MAX / 2 || splits < 1 || splits > 64 || K % splits)
+    return 0;
+  const int64_t ld_scale = wformat == B_MXFP8 ? K / 32 : 0;
+  const bool kg = splits == 1 ? kg_auto(wformat, M, N, K, K, K, ld_scale)
+                              : kg_ok(wformat, M, N, K / splits, K, K, ld_scale);
+  return kg ? kg_rows(wformat, M, N, K, splits, nullptr) : 0;
 }
 
 extern "C" int64_t ltx_gemm_splitk_workspace_bytes(int64_t M, int64_t N, int64_t splits) {

@@ -22,7 +22,7 @@ _f32 = ctypes.c_float
 _vp = ctypes.c_void_p
 
 # name -> argtypes (every function returns int: a status, or for
-# ltx_gemm_auto_splits the split count)
+# ltx_gemm_auto_splits / _rows the choice)
 SIGNATURES: dict[str, list] = {
     "ltx_version": [],
     "ltx_device_clock_stamp": [_vp, _vp],
@@ -46,6 +46,7 @@ SIGNATURES: dict[str, list] = {
     "ltx_gemm_rowss_bf16": [_int, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _int, _i64,
                             _vp, _i64, _i64, _vp],
     "ltx_gemm_auto_splits": [_i64, _i64, _i64, _int],
+    "ltx_gemm_auto_rows": [_i64, _i64, _i64, _int, _int],
     "ltx_gemm_splitk_bf16": [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64, _vp, _i64,
                              _int, _vp, _i64, _vp],
     "ltx_gemm_splitk_w8a16_bf16": [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _i64,

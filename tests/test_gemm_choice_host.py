@@ -1,6 +1,6 @@
 """The library's automatic GEMM choices (host code of csrc/gemm.hip), without a
-GPU: split counts for every depth the entry points take, and the entry that
-linear() calls."""
+GPU: split counts for every depth the entry points take, the entry that
+linear() calls, and which products the mid-size kernel takes."""
 
 from __future__ import annotations
 
@@ -58,3 +58,19 @@ def test_explicit_128_tiles_still_split(gemm, monkeypatch, m, n, k, splits):
     (name, args), = calls
     assert name == ("ltx_gemm_splitk_bf16" if splits > 1 else "ltx_gemm_bf16")
     assert splits == 1 or args[15] == splits
+
+
+def _rows(gemm, m, n, k, kind, splits=1):
+    """Tile height of an automatic launch on the mid-size kernel, 0: another kernel."""
+    return gemm._lib.lib().ltx_gemm_auto_rows(m, n, k, gemm._WFORMAT[kind], splits)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_shallow_products_of_many_tiles_keep_the_older_kernels(gemm, kind):
+    """The latent projections (K = 128): the mid-size kernel only where its
+    64-row tiles are one round."""
+    for m, n in ((700, 4096), (1296, 4096), (1728, 4096), (1296, 2048)):
+        assert _rows(gemm, m, n, 128, kind) == 0 and _rows(gemm, m, n, 256, kind) == 0
+    if kind != "mxfp8":  # MXFP8: whole groups of 512
+        assert _rows(gemm, 700, 2048, 128, kind) == 64 and _rows(gemm, 68, 2048, 256, kind) == 64
+    assert _rows(gemm, 1296, 4096, 512, kind) > 0
