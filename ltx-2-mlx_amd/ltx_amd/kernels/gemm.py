@@ -413,8 +413,15 @@ def rowss_eligible(x: torch.Tensor, weight: LinearWeight) -> bool:
     return True
 
 
-def linear_rowss(x: torch.Tensor, weight: LinearWeight, ss_cols: int, *,
-                 sigmoid_from: int | None = None) -> tuple[torch.Tensor, torch.Tensor]:
+def single_g8_round(x: torch.Tensor, weight: LinearWeight) -> bool:
+    """Whether the product is one partial round of the 8-wave kernel (100-159
+    tiles of 256x256), where the automatic choice may be the mid-size kernel."""
+    m = x.numel() // max(weight.in_features, 1)
+    return rowss_eligible(x, weight) and ((m + 255) // 256) * ((weight.out_features + 255) // 256) < 160
+
+
+def linear_rowss(x: torch.Tensor, weight: LinearWeight, ss_cols: int, *, sigmoid_from: int | None = None,
+                 tile: int = TILE_AUTO) -> tuple[torch.Tensor, torch.Tensor]:
     """:func:`linear` with the bias epilogue on the 8-wave kernel, plus the
     per-row sums of squares of the bf16 outputs of columns [0, ss_cols) in
     fp32 partials of 64 columns: returns (out (M, N) bf16, ss (M, ss_cols/64)
@@ -429,7 +436,7 @@ def linear_rowss(x: torch.Tensor, weight: LinearWeight, ss_cols: int, *,
     out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     parts = ss_cols // 64
     ss = torch.empty((m, parts), dtype=torch.float32, device=x.device)
-    flags = EPI_BIAS
+    flags = EPI_BIAS | (tile << 8)
     if weight.qlinear and weight.bias is not None:
         flags |= _lib.GEMM_ROUND_THEN_BIAS
     sig = n if sigmoid_from is None else int(sigmoid_from)

@@ -83,7 +83,7 @@ class Attention:
 
     def core(self, x: torch.Tensor, context: torch.Tensor | None = None,
              pe: tuple | None = None, k_pe: tuple | None = None, passes: int = 1,
-             kv: torch.Tensor | None = None, kv_ready=None) -> torch.Tensor:
+             kv: torch.Tensor | None = None, kv_ready=None, q_tile: int = gemm.TILE_AUTO) -> torch.Tensor:
         """Everything up to (not including) ``to_out``; returns (passes*Tq, inner) bf16.
 
         x: (passes*Tq, query_dim) bf16 -- ``passes`` independent sequences of
@@ -96,7 +96,9 @@ class Attention:
         the context's keys and values from :meth:`context_kv` (instead of
         ``context``; its keys are already normalised and rotated);
         ``kv_ready``: an event the current stream waits for before the first
-        read of ``kv`` (after the query projection and norm).
+        read of ``kv`` (after the query projection and norm).  ``q_tile``:
+        tile choice of a cross-attention's query projection where it is one
+        partial round of the 8-wave kernel.
         """
         inner, heads = self.inner_dim, self.heads
         gate_cols = heads if self.gated else 0
@@ -116,10 +118,12 @@ class Attention:
             g = None if not self.gated else (g if g.shape[1] == gate_cols else g[:, :gate_cols])
             k_tab = pe
         else:
+            if not gemm.single_g8_round(x, self.proj_q):
+                q_tile = gemm.TILE_AUTO
             if fused:
-                qb, ss = gemm.linear_rowss(x, self.proj_q, inner, sigmoid_from=inner)
+                qb, ss = gemm.linear_rowss(x, self.proj_q, inner, sigmoid_from=inner, tile=q_tile)
             else:
-                qb = gemm.linear(x, self.proj_q, sigmoid_from=inner)
+                qb = gemm.linear(x, self.proj_q, sigmoid_from=inner, tile=q_tile)
             kvb = gemm.linear(context, self.proj_kv) if kv is None else kv
             q = qb[:, :inner]
             g = qb[:, inner:inner + gate_cols] if self.gated else None

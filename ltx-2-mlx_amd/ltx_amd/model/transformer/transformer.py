@@ -55,6 +55,15 @@ from .feed_forward import FeedForward
 from ...components.perturbations import BatchedPerturbationConfig  # noqa: F401  (the block's perturbation type)
 from .rope import LTXRopeType
 
+# The A2V query projection stays on the 8-wave kernel where it is one of its
+# partial rounds (3456 x 4096 -> 2080: 126 workgroups).  The mid-size kernel runs
+# it 62 instead of 72 us alone (MXFP8) but in two rounds on every CU, and the
+# audio stream's work beside it then waits: the 48-block step measured 86.9-87.2
+# against 87.4-87.5 ms, 85.2 / 85.8 and 92.8 / 93.4 on other cards (int8 99.3 /
+# 99.6, 105.0 / 105.7; 3168 tokens 88.1 / 88.5).  One choice for the serial and the
+# concurrent block keeps their outputs the same bits.
+A2V_Q_TILE = gemm.TILE_G8
+
 # Dispatch shims (transformer.py:85-110): with LTX_FUSED_ADALN=1 the block's
 # AdaLN uses the fused kernel's single rounding; by default the compiled
 # inline form, whose rms_norm output is bf16 before the modulation.  Both run
@@ -563,16 +572,18 @@ class BasicAVTransformerBlock:
                     as_a2v.record_stream(main)
             if rng == [(0, npass)]:
                 if kv_a2v is not None:
-                    o = self.audio_to_video_attn.core(vs_a2v, pe=vpe, passes=npass, kv=kv_a2v, kv_ready=ev_a)
+                    o = self.audio_to_video_attn.core(vs_a2v, pe=vpe, passes=npass, kv=kv_a2v, kv_ready=ev_a,
+                                                      q_tile=A2V_Q_TILE)
                 else:
-                    o = self.audio_to_video_attn.core(vs_a2v, as_a2v, pe=vpe, k_pe=ape, passes=npass)
+                    o = self.audio_to_video_attn.core(vs_a2v, as_a2v, pe=vpe, k_pe=ape, passes=npass,
+                                                      q_tile=A2V_Q_TILE)
                 v2 = residual_gemm(o, self.audio_to_video_attn.to_out, v2, v_owned, ada_v[ROW_GATE_AV],
                                    gemm.EPI_RESIDUAL)
                 v_owned = True
             elif rng:
                 def a2v(dst, src, p0, p1):
                     o = self.audio_to_video_attn.core(vs_a2v[p0 * tv:p1 * tv], as_a2v[p0 * ta:p1 * ta], pe=vpe,
-                                                      k_pe=ape, passes=p1 - p0)
+                                                      k_pe=ape, passes=p1 - p0, q_tile=A2V_Q_TILE)
                     gemm.linear(o, self.audio_to_video_attn.to_out, epilogue=gemm.EPI_RESIDUAL, out=dst,
                                 residual=src, gate=ada_v[ROW_GATE_AV])
                 v2 = partial_residual(v2, v_owned, tv, rng, a2v)
