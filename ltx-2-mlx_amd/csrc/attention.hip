@@ -765,11 +765,12 @@ __global__ __launch_bounds__(64 * WAVES, 8 / WAVES) void flash_attn_kernel(
 // Combine of the split-KV partials: one thread per (query, head, 8 outputs).
 // O = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s, m = max_s m_s; then the
 // same rounding and gate as the single-pass epilogue.  Bound by the latency
-// of its loads: four splits' go out together (their sums stay in split order)
-// and one-wave workgroups spread a few queries over all CUs.
-constexpr int kCombineThreads = 64;
+// of its loads: those of four splits go out together, then of two and of one
+// (their sums stay in split order; four loads for a remainder of two cost 68 x
+// 256 keys 8.2 -> 8.6 us with the attention), and one-wave workgroups spread a
+// few queries over all CUs.
 template <int DH, bool GATED>
-__global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(SplitOut so, bf16* __restrict__ O, int64_t o_rs,
+__global__ __launch_bounds__(256) void attn_combine_kernel(SplitOut so, bf16* __restrict__ O, int64_t o_rs,
                                                            const bf16* __restrict__ G, int64_t g_rs,
                                                            int Tq, int H) {
   constexpr int CH = DH / 8;
@@ -779,24 +780,35 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(SplitOut 
   const int64_t qh = i / CH;  // q * H + head
   const int q = (int)(qh / H), head = (int)(qh % H);
   const int64_t plane = (int64_t)Tq * H;
-  constexpr int B = 4;
+  // f(first split, batch size) over batches of four, two and one splits
+  auto batches = [&](auto f) __attribute__((always_inline)) {
+    int s0 = 0;
+    for (; s0 + 4 <= so.splits; s0 += 4) f(s0, std::integral_constant<int, 4>{});
+    if (so.splits & 2) {
+      f(s0, std::integral_constant<int, 2>{});
+      s0 += 2;
+    }
+    if (so.splits & 1) f(s0, std::integral_constant<int, 1>{});
+  };
   float m = -INFINITY;
-  for (int s0 = 0; s0 < so.splits; s0 += B) {
-    float ms[B];  // past the last split, its value again
+  batches([&](int s0, auto bc) __attribute__((always_inline)) {
+    constexpr int B = decltype(bc)::value;
+    float ms[B];
 #pragma unroll
-    for (int u = 0; u < B; ++u) ms[u] = so.m[(s0 + u < so.splits ? s0 + u : so.splits - 1) * plane + qh];
+    for (int u = 0; u < B; ++u) ms[u] = so.m[(s0 + u) * plane + qh];
 #pragma unroll
     for (int u = 0; u < B; ++u) m = fmaxf(m, ms[u]);
-  }
+  });
   float l = 0.0f, o[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) o[e] = 0.0f;
-  for (int s0 = 0; s0 < so.splits; s0 += B) {
+  batches([&](int s0, auto bc) __attribute__((always_inline)) {
+    constexpr int B = decltype(bc)::value;
     float ms[B], ls[B];
     f32x4 x[B][2];
 #pragma unroll
     for (int u = 0; u < B; ++u) {
-      const int64_t row = (s0 + u < so.splits ? s0 + u : so.splits - 1) * plane + qh;
+      const int64_t row = (s0 + u) * plane + qh;
       ms[u] = so.m[row];
       ls[u] = so.l[row];
       x[u][0] = *reinterpret_cast<const f32x4*>(so.o + row * DH + c * 8);
@@ -804,13 +816,12 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(SplitOut 
     }
 #pragma unroll
     for (int u = 0; u < B; ++u) {
-      if (s0 + u >= so.splits) break;
       const float w = ms[u] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ms[u] - m);
       l = fmaf(w, ls[u], l);
 #pragma unroll
       for (int e = 0; e < 8; ++e) o[e] = fmaf(w, x[u][e >> 2][e & 3], o[e]);
     }
-  }
+  });
   const float inv_l = 1.0f / l;
   float g = 1.0f;
   if (GATED) g = (float)G[(int64_t)q * g_rs + head];
@@ -1040,13 +1051,19 @@ static int launch_attn_splitkv(const void* Q, int64_t q_rs, const void* K, int64
                     (int)splits};
   const float scale_log2 = scale * 1.4426950408889634f;
   const int64_t cthreads = Tq * H * (head_dim / 8);
-  const int cblocks = (int)((cthreads + kCombineThreads - 1) / kCombineThreads);
+  // One-wave workgroups (68 queries of 68 CUs' worth of four-wave ones), and at
+  // head_dim 128 for any count: four-wave ones took 256 x 256 keys from 12.6 to
+  // 15.2 us with the attention, 512 x 256 from 15.1 to 20.6.  At head_dim 64 more
+  // than ~90 queries are faster in four-wave ones: 121 x 256 9.5 -> 9.0, 512 x
+  // 577 21.3 -> 19.9.
+  const int cwg = head_dim == 64 && cthreads > 24576 ? 256 : 64;
+  const int cblocks = (int)((cthreads + cwg - 1) / cwg);
 #define LTX_FAS(DH, G)                                                                              \
   do {                                                                                              \
     flash_attn_kernel<DH, false, kAttnSplitWaves, true, VROW><<<(int)nwg, 64 * kAttnSplitWaves, 0, s>>>( \
         (const bf16*)Q, q_rs, (const bf16*)K, k_rs, (const bf16*)V, v_ld, nullptr, 0, nullptr,      \
         0, (int)Tq, (int)Tk, (int)H, scale_log2, so, QNorm{});                                      \
-    attn_combine_kernel<DH, G><<<cblocks, kCombineThreads, 0, s>>>(so, (bf16*)O, o_rs, (const bf16*)gate,       \
+    attn_combine_kernel<DH, G><<<cblocks, cwg, 0, s>>>(so, (bf16*)O, o_rs, (const bf16*)gate,                   \
                                                        gate_rs, (int)Tq, (int)H);                    \
   } while (0)
   if (head_dim == 128) {

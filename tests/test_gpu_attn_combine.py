@@ -1,6 +1,7 @@
-"""The split-KV combine at split counts around its batches of four loads and
-query counts around its one-wave workgroups: against the single pass on the
-same inputs, and bit-identical between runs.
+"""The split-KV combine at split counts around its batches of four, two and one
+splits and query counts around its one- and four-wave workgroups (385 x 8 heads
+of 64: the first four-wave launch): against the single pass on the same inputs,
+and bit-identical between runs.
 
 Bound: both forms round P to bf16 once per key and the output once; they differ
 in the running maximum that P is scaled by, so by bf16 roundings of P
@@ -18,8 +19,8 @@ from _util import max_rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("splits", [2, 3, 4, 5, 8, 9])
-@pytest.mark.parametrize("tq,H,dh", [(1, 1, 64), (1, 2, 128), (9, 3, 64), (130, 2, 128)])
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("tq,H,dh", [(1, 1, 64), (1, 2, 128), (9, 3, 64), (130, 2, 128), (385, 8, 64)])
 def test_combine_matches_single_pass(splits, tq, H, dh):
     from ltx_amd.kernels import attention as A
 
