@@ -9,13 +9,15 @@
 // up to the kernel launch, which the HIP runtime refuses for want of a
 // device (LTX_ERR_HIP), so AddressSanitizer sees the launch planning too.
 // Device pointers are fake, 16-byte aligned addresses that the library must
-// never dereference on the host.
+// never dereference on the host.  The address arithmetic that kernels and host
+// share (csrc/gemm_addr.h) is enumerated as well.
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <initializer_list>
 
 #include "../../include/ltx_hip.h"
+#include "../csrc/gemm_addr.h"
 
 // the HIP runtime's device count (C ABI of libamdhip64, which the library links)
 extern "C" int hipGetDeviceCount(int* count);
@@ -29,6 +31,29 @@ static void expect(const char* what, int64_t got, int64_t want) {
   }
 }
 #define EXPECT(call, want) expect(#call, (int64_t)(call), (int64_t)(want))
+
+// Every 16-byte direct load of the GEMMs' stage pairs lies inside its row of
+// `stages` 64-byte stages, for any unit a ring asks for (past the last one too)
+// and an odd count, and brings the chunk that its slot stands for wherever that
+// chunk's stage exists.
+static void check_pair_loads() {
+  for (int stages = 1; stages <= 12; ++stages) {
+    const int units = ltx::stage_pairs(stages);
+    for (int ask = 0; ask < units + 4; ++ask) {
+      const int u = ltx::clamp_unit(ask, units);
+      bool seen[8][8] = {};
+      for (int lane = 0; lane < 64; ++lane) {
+        const int chunk = ltx::pair_chunk(lane), row = lane >> 3;
+        const int back = ltx::half_pair(u, stages) ? ltx::half_pair_back(lane) : 0;
+        const int off = chunk * 16 - back + u * 128;
+        EXPECT(off >= 0 && off + 16 <= stages * 64, 1);
+        if (2 * u + (chunk >> 2) < stages) EXPECT(off, u * 128 + chunk * 16);
+        EXPECT(chunk >= 0 && chunk < 8 && !seen[row][chunk], 1);  // the eight chunks of a row, each once
+        seen[row][chunk & 7] = true;
+      }
+    }
+  }
+}
 
 int main(int argc, char** argv) {
   if (argc > 1 && std::strcmp(argv[1], "--overflow-selftest") == 0) {
@@ -50,6 +75,8 @@ int main(int argc, char** argv) {
   EXPECT(ltx_version() > 0, 1);
   EXPECT(ltx_device_clock_stamp(nullptr, nullptr), LTX_ERR_INVALID_ARG);
   EXPECT(ltx_device_clock_stamp(reinterpret_cast<uint64_t*>(static_cast<char*>(m) + 4), nullptr), LTX_ERR_ALIGNMENT);
+
+  check_pair_loads();
 
   // row kernels
   EXPECT(ltx_adaln_norm_fused_bf16(nullptr, 4096, fd, fd, d, 4096, 4, 4096, 1e-6f, 0, nullptr), LTX_ERR_INVALID_ARG);

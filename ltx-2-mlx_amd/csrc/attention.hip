@@ -1051,7 +1051,7 @@ static int launch_attn_splitkv(const void* Q, int64_t q_rs, const void* K, int64
                     (int)splits};
   const float scale_log2 = scale * 1.4426950408889634f;
   const int64_t cthreads = Tq * H * (head_dim / 8);
-  // One-wave workgroups (68 queries of 68 CUs' worth of four-wave ones), and at
+  // One-wave workgroups (68 queries fill 68 CUs with four-wave ones), and at
   // head_dim 128 for any count: four-wave ones took 256 x 256 keys from 12.6 to
   // 15.2 us with the attention, 512 x 256 from 15.1 to 20.6.  At head_dim 64 more
   // than ~90 queries are faster in four-wave ones: 121 x 256 9.5 -> 9.0, 512 x

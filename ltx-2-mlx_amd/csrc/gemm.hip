@@ -825,8 +825,9 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // registers), a fixed 32-bit per-lane byte offset in one vector register,
   // the stage's advance as the scalar offset and the LDS destination in M0
   // -- no vector instructions per load (vector instructions of one wave take
-  // matrix-pipe slots from the other).  The descriptors' record counts bound
-  // every load to its operand (g8_ok checks the 32-bit extents).
+  // matrix-pipe slots from the other).  The descriptors' record counts bound the
+  // lane offsets to their operand (g8_ok checks the 32-bit extents), the clamps
+  // on the stage the scalar offset, which the counts do not cover.
   const int a_records = (int)((int64_t)p.M * p.lda * (MX ? 1 : 2)),
             b_records = (int)(((int64_t)(p.N - 1) * p.ldb + p.K) * (BF ? 2 : 1));
   const int loader = W8 ? wave & 3 : wave;
@@ -844,7 +845,7 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
       const int r = 8 * (LOADERS * d + loader) + (lane >> 3);
       int gm = m0 + r;
       gm = gm < p.M ? gm : p.M - 1;
-      const int chunk = (lane & 7) ^ (BF ? swz_pair(r) : g8_swz128(r, S16));
+      const int chunk = BF ? pair_chunk(lane) : (lane & 7) ^ g8_swz128(r, S16);
       a_src[d] = (uint32_t)((int64_t)gm * p.lda * 2) + chunk * 16;
     }
   }
@@ -854,25 +855,23 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
     const int r = MX ? 16 * (8 * d + wave) + (lane >> 2) : 8 * (LOADERS * d + loader) + (lane >> 3);
     int gn = n0 + r;
     gn = gn < p.N ? gn : p.N - 1;
-    const int chunk = MX ? (lane & 3) ^ g8_swz64(r, S16) : (lane & 7) ^ swz_pair(r);
+    const int chunk = MX ? (lane & 3) ^ g8_swz64(r, S16) : pair_chunk(lane);
     b_src[d] = (uint32_t)((int64_t)gn * p.ldb * (BF ? 2 : 1)) + chunk * 16;
   }
-  // the activations' stage (BF: pair) `u` / the weights' pair, clamped to the
-  // last one, into ring slot `slot`.  In a last half pair (int8, odd KT) the
-  // lanes of the missing stage read the other one's bytes again, so that no
-  // load leaves its row (the record count does not bound the scalar offset).
-  const int last_a = BF ? (KT >> 1) - 1 : KT - 1, last_b = ((KT + 1) >> 1) - 1;
+  // the activations' stage (BF: pair) `u` / the weights' pair into ring slot
+  // `slot`; gemm_addr.h keeps every load inside its row
+  const int a_units = BF ? KT >> 1 : KT, b_units = stage_pairs(KT);
   auto dma_a = [&](int u, int slot) __attribute__((always_inline)) {
-    u = u < last_a ? u : last_a;
+    u = clamp_unit(u, a_units);
 #pragma unroll
     for (int d = 0; d < A_DMA; ++d)
       buffer_dma16(p.A, a_records, a_src[d], u * A_ROWB, lds + slot * A_BYTES + (LOADERS * d + loader) * 1024);
   };
   auto dma_b = [&](int u, int slot) __attribute__((always_inline)) {
-    u = u < last_b ? u : last_b;
-    if constexpr (BKIND == B_INT8) {
-      if (u == last_b && (KT & 1)) {
-        const uint32_t back = (((lane & 7) ^ swz_pair(lane >> 3)) & 4) * 16;
+    u = clamp_unit(u, b_units);
+    if constexpr (BKIND == B_INT8) {  // bf16: 32-deep stages, MXFP8: whole octets -- always even counts
+      if (half_pair(u, KT)) {
+        const uint32_t back = half_pair_back(lane);
 #pragma unroll
         for (int d = 0; d < B_DMA; ++d)
           buffer_dma16(p.B, b_records, b_src[d] - back, u * B_ROWB,

@@ -5,6 +5,7 @@
 
 #include <type_traits>
 
+#include "gemm_addr.h"
 #include "ltx_common.h"
 
 namespace ltx {
@@ -192,12 +193,6 @@ __device__ __forceinline__ int g8_swz64(int r, bool s16) { return s16 ? ((r & 1)
 __device__ __forceinline__ int g8_swz128(int r, bool s16) {
   return s16 ? (((r >> 1) & 1) | ((r & 1) << 1) | (r & 4)) : ((r >> 1) & 7);
 }
-
-// The same for a 128-byte row that holds two 64-byte halves of 16x16 fragment
-// reads (chunk 4 half + q of rows r16): a lane-octet pair that is served
-// together holds eight rows at q and eight at q ^ 1, and even rows keep chunk
-// bit 0, so the pair covers all 64 banks.
-__device__ __forceinline__ int swz_pair(int r) { return r & 6; }
 
 // gemm_kg.hip: launch the mid-size kernel with BM-row tiles (64, 128 or 192)
 // and `splits` K ranges (epi kEpiPartial; p.K is then the depth of one).

@@ -124,14 +124,16 @@ __global__ __launch_bounds__(kKgThreads, 1) void gemm_kg_kernel(GemmArgs p) {
   // groups' halves, so every row of a load is a whole 128-byte line: half
   // lines cost the L2 as many requests each.  8-bit weights' activations, 128
   // bytes per group, are group 0's rows, then group 1's.  Rows past M / N
-  // re-read the last row; the record counts bound every load to its operand.
+  // re-read the last row.  The record counts bound the lane offsets to their
+  // operand; the scalar offset, which they do not cover, stays inside the row
+  // because past the last unit that one is loaded again.
   const int a_records = (int)((int64_t)p.M * p.lda * 2), b_records = (int)((int64_t)p.N * p.ldb * ES);
   uint32_t a_src[A_DMA];
 #pragma unroll
   for (int d = 0; d < A_DMA; ++d) {
     const int lr = 8 * (8 * d + wave) + (lane >> 3);  // LDS row
     const int r = BF ? lr : lr % BM, g = BF ? 0 : lr / BM;
-    const int chunk = (lane & 7) ^ (BF ? swz_pair(r) : g8_swz128(r, true));
+    const int chunk = BF ? pair_chunk(lane) : (lane & 7) ^ g8_swz128(r, true);
     int gm = m0 + r;
     gm = gm < p.M ? gm : p.M - 1;
     a_src[d] = (uint32_t)(((int64_t)gm * p.lda + k0) * 2) + g * 128 + chunk * 16;
@@ -140,10 +142,9 @@ __global__ __launch_bounds__(kKgThreads, 1) void gemm_kg_kernel(GemmArgs p) {
 #pragma unroll
   for (int d = 0; d < B_DMA; ++d) {
     const int r = 8 * (8 * d + wave) + (lane >> 3);
-    const int chunk = (lane & 7) ^ swz_pair(r);
     int gn = n0 + r;
     gn = gn < p.N ? gn : p.N - 1;
-    b_src[d] = (uint32_t)(((int64_t)gn * p.ldb + k0) * ES) + chunk * 16;
+    b_src[d] = (uint32_t)(((int64_t)gn * p.ldb + k0) * ES) + pair_chunk(lane) * 16;
   }
   // MXFP8 scales, four units at a time: 16 bytes per weight row, a dword per
   // lane of 16 rows per wave (a dword per unit of 64 rows per wave would
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(kKgThreads, 1) void gemm_kg_kernel(GemmArgs p) {
   // the last unit, data that nobody reads
   constexpr int NL = A_DMA + B_DMA;
   auto load = [&](int u, int sa, int sb, int l) __attribute__((always_inline)) {
-    const int ua = u + RA < KT ? u + RA : KT - 1, ub = u + RB < KT ? u + RB : KT - 1;
+    const int ua = clamp_unit(u + RA, KT), ub = clamp_unit(u + RB, KT);
     if (l < A_DMA)
       buffer_dma16(p.A, a_records, a_src[l < A_DMA ? l : 0], ua * 4 * Cfg::KU,
                    lds + sa * 2 * A_BYTES + (8 * l + wave) * 1024);

@@ -1,8 +1,9 @@
 """The 8-wave kernel's rings of stage pairs (csrc/gemm.hip): identity products,
-exact (one product 1.0 * w per output), at the depths where the pairs can go
-wrong -- one stage, an odd stage count (half a pair of int8 codes), every
-remainder of a ring turn -- with both tile heights and weights whose rows end
-at the end of their buffer (a load past it would bring other bytes).
+exact (one product 1.0 * w per output), at the depths where the order of the
+rings can go wrong -- one stage, an odd stage count (half a pair of int8 codes),
+every remainder of a ring turn -- with both tile heights and strided weights.
+That no load leaves its row is not visible in outputs (the bytes of a missing
+stage are never multiplied); the host checks enumerate the addresses.
 """
 
 from __future__ import annotations
