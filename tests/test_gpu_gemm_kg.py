@@ -1,12 +1,13 @@
 """The mid-size projection kernel (csrc/gemm_kg.hip) through the automatic
-tile choice, at the edges of its tiles: every tile height (64, 128, 192 rows),
-one row, partial tiles in both directions, a wave tile wholly past M or N, the
-fewest units of its rings (K = 128 bf16 / int8, 512 MXFP8) and an odd number
-of units, and its split-K form.
+tile choice, at the edges of its tiles: each tile height (64, 128, 192 rows; the
+test asks the library that its shape gets it), one row past a tile, half a tile
+and one row more (a wave tile wholly past M or N), the fewest units of its rings
+and counts that are no multiple of four, single pass and split-K.
 
-Bounds: the in-GEMM dequantisation and an identity product are exact (one
-product 1.0 * w per output); the epilogues match the oracle at the GEMM gate
-of test_gpu_gemm.py (bf16 outputs of fp32 sums in another order).
+Bounds: the in-GEMM dequantisation, an identity product (one product 1.0 * w per
+output) and products of small whole numbers (every partial sum is exact) are
+exact; the epilogues match the oracle at the GEMM gate of test_gpu_gemm.py (bf16
+outputs of fp32 sums in another order).
 """
 
 from __future__ import annotations
@@ -68,6 +69,55 @@ def test_epilogues(kind, epi, M, K, N, splits):
     if sig is not None:
         ref[:, sig:] = oq.linear(x, _decoded(kind, W), b, epilogue="sigmoid2", round_then_bias=qlin)[:, sig:]
     _check(bf16_from_torch(out), ref, min_exact=0.85)
+
+
+def _whole(rng, shape, lo, hi):
+    return rng.integers(lo, hi + 1, shape).astype(np.float32)
+
+
+# (tile height, splits, M, N): M one row, half a tile or half a tile and one row
+# past whole tiles, N 8 or 72 columns past 128
+HEIGHTS = [(64, 1, 1, 72), (64, 1, 33, 136), (64, 2, 32, 72), (64, 4, 65, 264),
+           (128, 1, 385, 4680), (128, 1, 3392, 520), (128, 1, 449, 4168),
+           (128, 2, 257, 3272), (128, 2, 2752, 264), (128, 4, 129, 2760), (128, 4, 2112, 200), (128, 4, 65, 4104),
+           (192, 1, 769, 4680), (192, 1, 1056, 3656), (192, 1, 1057, 3656),
+           (192, 2, 385, 4168), (192, 2, 5472, 264), (192, 4, 385, 2120), (192, 4, 288, 2760), (192, 4, 4129, 136)]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("depth", ["fewest", "odd"])
+@pytest.mark.parametrize("bm,splits,M,N", HEIGHTS)
+def test_each_tile_height_at_its_edges(bm, splits, M, N, depth, kind):
+    """Whole-number operands: x in [-1, 2], weights that each format holds
+    exactly, so outputs are the oracle's bits in any order of the sums.
+    ``odd``: 10 (bf16), 5 (int8) or 12 (MXFP8) units; ``fewest``: 2, 1 or 4
+    (in a single pass of the taller tiles 8, 4 or 4: below, other kernels)."""
+    from ltx_amd import _lib
+    from ltx_amd.kernels import gemm
+
+    per = {"odd": (640, 1536), "fewest": (128 if splits > 1 or bm == 64 else 512, 512)}[depth][kind == "mxfp8"]
+    K = per * splits
+    assert _lib.lib().ltx_gemm_auto_rows(M, N, K, gemm._WFORMAT[kind], splits) == bm
+    print(f"{kind} {M} x {K} -> {N} rows {bm} splits {splits}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    x, W = _whole(rng, (M, K), -1, 2), _whole(rng, (N, K), -4, 4)
+    if kind == "int8":  # 127 in every row: a scale of exactly one
+        W[:, 0] = 127.0
+    b, res = _whole(rng, N, -8, 8), _whole(rng, (M, N), -64, 64)
+    gate = np.float32(0.5) * np.ones(N, np.float32)
+    np.testing.assert_array_equal(_decoded(kind, W), W)
+    wt = gemm.make_weight(_t(W), _t(b, torch.float32), kind=kind)
+    buf = torch.full((M + 2, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = buf[:M, :N]
+    qlin = kind == "mxfp8"
+    gemm.linear(_t(x), wt, out=out, splits=splits)
+    ref = oq.linear(x, W, b, epilogue="bias", round_then_bias=qlin)
+    np.testing.assert_array_equal(bf16_from_torch(out), ref)
+    gemm.linear(_t(x), wt, epilogue=gemm.EPI_RESIDUAL, out=out, residual=_t(res), gate=_t(gate, torch.float32),
+                splits=splits)
+    ref = oq.linear(x, W, b, epilogue="residual", residual=res, gate=gate, round_then_bias=qlin)
+    np.testing.assert_array_equal(bf16_from_torch(out), ref)
+    assert (buf[M:] == 7.0).all() and (buf[:, N:] == 7.0).all()
 
 
 @pytest.mark.parametrize("kind", KINDS)
