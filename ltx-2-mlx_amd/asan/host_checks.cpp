@@ -22,6 +22,13 @@
 // the HIP runtime's device count (C ABI of libamdhip64, which the library links)
 extern "C" int hipGetDeviceCount(int* count);
 
+// gemm_kg.hip's launcher (library-internal): refuses what it has no kernel for
+struct ihipStream_t;
+namespace ltx {
+struct GemmArgs;
+bool kg_launch(int bkind, const GemmArgs& p, int epi, int bm, int splits, ::ihipStream_t* s);
+}  // namespace ltx
+
 static int failures = 0;
 
 static void expect(const char* what, int64_t got, int64_t want) {
@@ -77,6 +84,10 @@ int main(int argc, char** argv) {
   EXPECT(ltx_device_clock_stamp(reinterpret_cast<uint64_t*>(static_cast<char*>(m) + 4), nullptr), LTX_ERR_ALIGNMENT);
 
   check_pair_loads();
+  static const char no_args[1024] = {};  // never read: refused before
+  const ltx::GemmArgs& none = *reinterpret_cast<const ltx::GemmArgs*>(no_args);
+  EXPECT(ltx::kg_launch(0, none, 5, 64, 1, nullptr), 0);  // the MX kernel's epilogue
+  EXPECT(ltx::kg_launch(3, none, 0, 64, 1, nullptr), 0);  // quantised activations
 
   // row kernels
   EXPECT(ltx_adaln_norm_fused_bf16(nullptr, 4096, fd, fd, d, 4096, 4, 4096, 1e-6f, 0, nullptr), LTX_ERR_INVALID_ARG);

@@ -1571,8 +1571,7 @@ template <int BKIND, int EPI>
 static int launch_epi_w(const GemmArgs& p, int tile, hipStream_t s) {
   const bool auto_tile = tile == 0;
   if (auto_tile && kg_auto(BKIND, p.M, p.N, p.K, p.lda, p.ldb, p.ld_scale)) {
-    kg_launch(BKIND, p, EPI, kg_rows(BKIND, p.M, p.N, p.K, 1, nullptr), 1, s);
-    return LTX_OK;
+    return kg_launch(BKIND, p, EPI, kg_rows(BKIND, p.M, p.N, p.K, 1, nullptr), 1, s) ? LTX_OK : LTX_ERR_UNSUPPORTED;
   }
   if (tile == 0) {
     // Large tiles when they still give most CUs a tile; 128x128 otherwise.
@@ -1740,11 +1739,13 @@ static int launch_splitk(const GemmArgs& p0, int epilogue, int splits, float* wo
   q.ldc = p.N;
   q.tiles_m = (p.M + 127) / 128;
   q.tiles_n = (p.N + 127) / 128;
-  if (tile == 0 && kg_ok(BKIND, q.M, q.N, q.K, q.lda, q.ldb, q.ld_scale))
-    kg_launch(BKIND, q, kEpiPartial, kg_rows(BKIND, p.M, p.N, p.K, splits, nullptr), splits, s);
-  else
+  if (tile == 0 && kg_ok(BKIND, q.M, q.N, q.K, q.lda, q.ldb, q.ld_scale)) {
+    if (!kg_launch(BKIND, q, kEpiPartial, kg_rows(BKIND, p.M, p.N, p.K, splits, nullptr), splits, s))
+      return LTX_ERR_UNSUPPORTED;
+  } else {
     gemm_kernel<128, 128, 64, 2, BKIND, kEpiPartial, 0, LOAD_REG>
         <<<q.tiles_m * q.tiles_n * splits, kGemmThreads, 0, s>>>(q);
+  }
   // pass 2: sum + epilogue
   p.partial = workspace;
   const int64_t vecs = (int64_t)p.M * (p.N / 8);
