@@ -314,9 +314,10 @@ int ltx_gemm_mxfp8_bf16(const void* A, int64_t lda, const uint8_t* Wq, int64_t l
  * outputs in columns [0, ss_cols):
  *   rowss[m * ld_rowss + j] = sum_{n in [64 j, 64 j + 64)} C[m, n]^2 (fp32).
  * ss_cols % 64 == 0, ss_cols <= min(N, sigmoid_from), ld_rowss >= ss_cols / 64,
- * rowss 4-byte aligned.  Always the eight-wave kernel (LTX_ERR_UNSUPPORTED
- * where it does not apply); C equals the plain entry point's result on that
- * kernel bit for bit.  No counterpart in the reference: the row statistics of
+ * rowss 4-byte aligned.  Without a tile code, the mid-size kernel where the plain
+ * entry points' automatic choice takes it, else the eight-wave kernel
+ * (LTX_ERR_UNSUPPORTED where that does not apply); C equals the plain entry
+ * point's result on the same kernel bit for bit.  No counterpart in the reference: the row statistics of
  * the query RMS norm (attention.py:578-580) for ltx_flash_attn_qnorm_v_bf16,
  * which then needs no separate pass over Q. */
 int ltx_gemm_rowss_bf16(int wformat, const void* A, int64_t lda, const void* W, int64_t ldw,

@@ -135,7 +135,7 @@ struct GemmArgs {
   int64_t ld_cscale;
   int M, N, K;         // split-K: K is the per-split depth
   int tiles_m, tiles_n;
-  // 8-wave bias epilogue: per-row sums of squares of the bf16 outputs of
+  // 8-wave and mid-size bias epilogue: per-row sums of squares of the bf16 outputs of
   // columns [0, ss_cols), one fp32 partial per 64-column slice at
   // rowss[row * ld_rowss + col / 64] (null: none)
   float* rowss = nullptr;

@@ -397,10 +397,13 @@ def _mx_eligible(m: int, n: int, k: int, weight: LinearWeight, tile: int) -> boo
 def rowss_eligible(x: torch.Tensor, weight: LinearWeight) -> bool:
     """Whether :func:`linear_rowss` takes this product: bf16 activations,
     weights of one of the three formats, at least 100 tiles of 256x256 (where
-    the automatic choice of :func:`linear` is the 8-wave kernel for a
-    projection at least as wide as half its depth, so both give the same
-    outputs) and the 8-wave kernel's conditions (MXFP8 weights: K a multiple
-    of 512), outside the opt-in MX path."""
+    the automatic choice is the 8-wave or the mid-size kernel, whose epilogues
+    give the statistics, and the same one for :func:`linear`) and the 8-wave
+    kernel's conditions (MXFP8 weights: K a multiple of 512), outside the
+    opt-in MX path.  Not bf16 products of 160 tiles on with fewer columns than
+    K (the A2V query projection of long clips): the attention with its norm
+    inside measured slower than with the separate pass (6144 x 68 tokens 144
+    against 138 us, 14640 x 68 324 against 316)."""
     if isinstance(x, MxRows) or x.dtype != torch.bfloat16 or weight.kind not in ("bf16", "int8", "mxfp8"):
         return False
     k, n = weight.in_features, weight.out_features
@@ -422,11 +425,11 @@ def single_g8_round(x: torch.Tensor, weight: LinearWeight) -> bool:
 
 def linear_rowss(x: torch.Tensor, weight: LinearWeight, ss_cols: int, *, sigmoid_from: int | None = None,
                  tile: int = TILE_AUTO) -> tuple[torch.Tensor, torch.Tensor]:
-    """:func:`linear` with the bias epilogue on the 8-wave kernel, plus the
-    per-row sums of squares of the bf16 outputs of columns [0, ss_cols) in
+    """:func:`linear` with the bias epilogue on the mid-size or the 8-wave
+    kernel (the automatic choice, or ``tile``), plus the per-row sums of squares of the bf16 outputs of columns [0, ss_cols) in
     fp32 partials of 64 columns: returns (out (M, N) bf16, ss (M, ss_cols/64)
     fp32) (ltx_gemm_rowss_bf16).  ``out`` is bit-identical to :func:`linear`
-    on that kernel."""
+    with the same ``tile`` (and one split)."""
     k = weight.in_features
     n = weight.out_features
     if not rowss_eligible(x, weight):

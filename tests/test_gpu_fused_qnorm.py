@@ -1,8 +1,9 @@
 """GPU parity of the query RMS norm + RoPE fused into the attention kernel.
 
 * ``ltx_gemm_rowss_bf16``: the projection output is bit-identical to
-  ``ltx_gemm_*`` (the 8-wave kernel, the automatic choice at these shapes),
-  and each row statistic equals the float64 sum of squares of those bf16
+  ``ltx_gemm_*`` (the automatic choice between the 8-wave and the mid-size
+  kernel, and the 8-wave kernel by request; the two agree within the GEMM
+  gate), and each row statistic equals the float64 sum of squares of those bf16
   outputs over its 64 columns within fp32 summation error.
 * ``ltx_flash_attn_qnorm_v_bf16`` on the raw projection against the separate
   in-place pass (``ltx_qknorm_rope_*``, pinned to the oracle in
@@ -65,6 +66,35 @@ def test_gemm_rowss_output_and_statistics(kind, M, N, ss_cols):
     assert ss.shape == (M, ss_cols // 64)
     rel = ((ss.double() - want).abs() / want.clamp_min(1e-30)).max().item()
     assert rel <= 64 * 2.0 ** -24, rel
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8", "mxfp8"])
+@pytest.mark.parametrize("M", [2848, 3456])
+def test_gemm_rowss_on_both_kernels(kind, M):
+    """The A2V query projection, one round of 192-row tiles (2848 rows) and two
+    of 128-row tiles (3456: MXFP8 and int8) of the mid-size kernel by the
+    automatic choice, one partial round of the 8-wave kernel by request.
+    The kernels add K in different orders: bf16 outputs within the GEMM gate."""
+    from ltx_amd import _lib
+    from ltx_amd.kernels import gemm
+
+    rng = np.random.default_rng(M)
+    N, K, ss_cols = 2080, 4096, 2048
+    x = _t(_bf(rng, (M, K)))
+    wt = gemm.make_weight(_t(_bf(rng, (N, K), 0.02)), _t(rng.standard_normal(N).astype(np.float32) * 0.02,
+                                                        torch.float32), kind=kind)
+    rows = _lib.lib().ltx_gemm_auto_rows(M, N, K, gemm._WFORMAT[kind], 1)
+    assert rows == (192 if M == 2848 else 0 if kind == "bf16" else 128)
+    outs = []
+    for tile in (gemm.TILE_AUTO, gemm.TILE_G8):
+        print(f"rowss {kind} M={M} tile={tile}", flush=True)
+        out, ss = gemm.linear_rowss(x, wt, ss_cols, sigmoid_from=ss_cols, tile=tile)
+        ref = gemm.linear(x, wt, sigmoid_from=ss_cols, tile=tile)
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+        want = (out[:, :ss_cols].double() ** 2).view(M, ss_cols // 64, 64).sum(-1)
+        assert ((ss.double() - want).abs() / want.clamp_min(1e-30)).max().item() <= 64 * 2.0 ** -24
+        outs.append(bf16_from_torch(out))
+    assert max_rel_err(*outs) <= 1e-2 and cos_sim(*outs) >= 0.9999
 
 
 def _grid_q(rng, shape):
