@@ -673,9 +673,10 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_kernel(GemmArgs p) {
 // group 0 (waves 0-3) owns output rows 0-127 of the tile, group 1 (waves 4-7)
 // rows 128-255; wave w & 3 owns 64 output columns.  The groups run half a
 // stage apart: while one group issues its memory cluster (LDS fragment reads
-// of a stage, its direct global->LDS loads of later stages, the scale loads), the other group's compute cluster (the stage's 64 16x16x32
-// MFMAs with the weight dequantisation of fragments 2-7 interleaved) keeps
-// the SIMD's matrix pipe busy.  The memory cluster ends, once its fragment
+// of a stage, its direct global->LDS loads of later stages, the scale loads),
+// the other group's compute cluster (the stage's 64 16x16x32 MFMAs with the
+// weight dequantisation of fragments 2-7 interleaved) keeps the SIMD's matrix
+// pipe busy.  The memory cluster ends, once its fragment
 // reads have landed, by decoding the stage's E8M0 scales and dequantising
 // fragments 0 and 1, so the compute cluster's first MFMAs issue right after
 // the barrier (FF up 402 -> 382 us: the dependent decode -> convert chain had
@@ -686,13 +687,14 @@ __global__ __launch_bounds__(kGemmThreads, 1) void gemm_kernel(GemmArgs p) {
 // one stage ahead, and pairs of stages of raw weight codes (256 x 128 B),
 // moved by group 1 with the scales a pair ahead, two slots each (all that fits
 // beside the scales; against three single stages, 64 bytes of codes per row,
-// moved by all waves: FF up 331 -> 326 us, QKV 258 -> 252, 6144 x 4096 ->
-// 12320 438 -> 428, 3888 x 16384 -> 4096 349 -> 341).  The MXFP8 / int8 codes are dequantised per fragment with the
-// exact format arithmetic, so the bf16 MFMA sees bit-exact weights.  bf16
-// weights: 32-deep stages that reach LDS in pairs (128-byte rows of both
-// operands), 32 MFMAs per cluster, no dequantisation; 64-byte rows, twice the
-// L2 requests, measured 390 against 350 us on FF up at M = 3456, 294 against
-// 267 on QKV, 228 against 200 on 2048 x 4096 -> 16384.
+// moved by all waves: FF up 329 -> 321 us, QKV 250 -> 244, 6144 x 4096 -> 12320
+// 428 -> 420, 3888 x 16384 -> 4096 340 -> 333; int8 FF up 383 -> 377).  The MXFP8
+// / int8 codes are dequantised per fragment with the exact format arithmetic, so
+// the bf16 MFMA sees bit-exact weights.  bf16 weights: 32-deep stages that reach
+// LDS in pairs (128-byte rows of both operands), 32 MFMAs per cluster, no
+// dequantisation; 64-byte rows, twice the L2 requests, measured 354 against 326
+// us on FF up at M = 3456, 267 against 248 on QKV, 197 against 184 on 2048 x 4096
+// -> 16384.
 // MX (8-bit codes of both operands): 16 scaled 32x32x64 MFMAs per cluster.
 //
 // Inside a stage the k order of the MFMA slots is permuted so that a lane
@@ -709,9 +711,10 @@ struct G8Cfg {
   static constexpr bool MX = BKIND == B_MX;
   // bf16 weights: stages are 32 deep, but both operands reach LDS in pairs of
   // stages, rows of 128 bytes: a 64-byte piece costs the L2 a request like a
-  // whole line does, and at two per line the requests kept its channels 0.7
-  // busy.  Rings of A_PAIRS and B_PAIRS pairs -- all that 160 KB hold: the
-  // activations (mostly L2 hits) one pair ahead, the weights (HBM) two.
+  // whole line does (FF up in 64-byte rows: 52 M requests in the 256-row
+  // launch, 0.70 per L2 channel and cycle; 27 M and 0.39 here).  Rings of A_SLOTS and B_SLOTS
+  // pairs -- all that 160 KB hold: the activations (mostly L2 hits) one pair
+  // ahead, the weights (HBM) two.
   static constexpr bool BF = BKIND == B_BF16;
   static constexpr int BM = BM_, BN = 256, BK = BF ? 32 : 64;
   // 8-bit weights (W8): the codes in pairs of 64-deep stages too (activation
@@ -819,8 +822,9 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // block of LDS, lane j its 16-byte slot j; the lane's source address picks
   // the logical chunk that the slot holds under the XOR swizzle of its row
   // (g8_swz128 for the 128-byte A rows, 8 per block; g8_swz64 for the 64-byte
-  // rows, 16 per block; swz_pair for BF's rows of a stage pair), the one under
-  // which this kernel's fragment reads are conflict-free.  Rows past M / N re-read the last row.
+  // rows, 16 per block; swz_pair for rows of a stage pair), the one under which
+  // this kernel's fragment reads are conflict-free.  Rows past M / N re-read the
+  // last row.
   // Direct loads as buffer loads: a buffer descriptor per operand (scalar
   // registers), a fixed 32-bit per-lane byte offset in one vector register,
   // the stage's advance as the scalar offset and the LDS destination in M0
@@ -908,12 +912,12 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
     a_mx[pp] = (wm * WM + fr) * A_ROWB + (((2 * pp + h) ^ b_swz) * 16);
   }
   // 16x16x32 fragments: lane (r16, q) = row r16 of a 16-row block, k-quarter
-  // q.  Weights: one 16-byte read per block and stage, chunk q of the 64-byte
-  // row (8-bit codes: k = 16 q + [0, 16), both k-steps).  8-bit codes: k-step s of the stage is
-  // k = 16 q + 8 s + [0, 8) in lane q for both operands -- the activation
-  // fragment is chunk 2 q + s of the 128-byte row -- so the E8M0 block of a
-  // lane's codes is q / 2 in both k-steps.  Every 16 lanes read 16
-  // consecutive rows of one logical chunk (conflict-free under g8_swz64 /
+  // q.  Weights: one 16-byte read per block and stage, chunk q of the stage's
+  // half row (8-bit codes: k = 16 q + [0, 16), both k-steps).  8-bit codes:
+  // k-step s of the stage is k = 16 q + 8 s + [0, 8) in lane q for both operands
+  // -- the activation fragment is chunk 2 q + s of the 128-byte row -- so the
+  // E8M0 block of a lane's codes is q / 2 in both k-steps.  Every 16 lanes read
+  // 16 consecutive rows of one logical chunk (conflict-free under swz_pair and
   // g8_swz128 of the 16x16 form; the row's bits 0-3 are those of r16).
   // The activation bases come as a low / high pair (stage buffers 0-1 / 1-2
   // of the 8-bit-code ring) so that the offsets fit the 16-bit immediate.
@@ -934,8 +938,8 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // make the compiler wait for every load in flight (its wait counting does
   // not see the direct loads).  Octet o of a tile is 256 weight rows x 16
   // bytes (the E8M0 of k-blocks 16o..16o+15, i.e. stages 8o..8o+7), laid out
-  // [row][16]; waves 0-3 each move 64 rows per octet.  int8: the row scale
-  // in a register.
+  // [row][16]; the four waves of group 1, which moves the codes, take 64 rows
+  // per octet each.  int8: the row scale in a register.
   // MX: group 0 moves the weights' octets, group 1 the activations' (256
   // activation rows x 16 bytes, after the weights' two octet buffers).
   char* const sc_lds = lds + Cfg::SC_OFF;
@@ -1181,7 +1185,8 @@ __global__ __launch_bounds__(kG8Threads, 1) void gemm8_kernel(GemmArgs p) {
   // leaving only the loads of later stages in flight.  Past the last stage the
   // direct loads re-read the last one into the buffer nobody reads any more,
   // so every stage issues the same loads and the waits are exact.  The scales
-  // of octet o+1 go out (group 0) with stage 8o's loads.
+  // of octet o+1 go out with stage 8o's loads (8-bit weights: by group 1; MX:
+  // by both groups, an operand each).
   // BF: the memory cluster of a pair's first stage issues the activations'
   // next free pair, that of its second stage the weights'; only the last
   // stage of a pair waits, for the next pair.
@@ -1574,25 +1579,20 @@ static int launch_epi_w(const GemmArgs& p, int tile, hipStream_t s) {
     return kg_launch(BKIND, p, EPI, kg_rows(BKIND, p.M, p.N, p.K, 1, nullptr), 1, s) ? LTX_OK : LTX_ERR_UNSUPPORTED;
   }
   if (tile == 0) {
-    // Large tiles when they still give most CUs a tile; 128x128 otherwise.
-    // 8-bit weights take the 8-wave kernel from 100 tiles of 256x256: the A2V
-    // query projection (3456 x 4096 -> 2048, 112 tiles) runs in 76 instead of
-    // 86 us alone, and the step gains 0.6-0.7 ms (the CUs its single round
-    // leaves free take the audio stream's work).  (256x128 tiles, 14 % faster
-    // on that projection alone, were 0.25 ms slower per step: explicit only.)
-    // int8 measured faster there than on the 4-wave kernel on every block
-    // shape (4096^2 109 vs 134 us, FF up 428 vs 472, FF down 405 vs 435).
-    // (128-row tiles for the A2V query projection, 126 -> 243 tiles: 79 ->
-    // 61 us alone, but the step 1.0-1.6 ms slower in two A/B pairs -- 48 %
-    // more CU time per launch, which the audio stream's work beside it then
-    // lacks: explicit only, LTX_GEMM_TILE_G8_128.)
-    // bf16 weights take it too: faster than the 4-wave kernel on every shape
-    // of 100 tiles on (FF up 350 vs 420 us, 4096^2 91 vs 105, FF down 339 vs
-    // 404, 1024 x 4096 -> 12320 87 vs 101).
+    // What the mid-size kernel does not take: large tiles when they still give
+    // most CUs a tile, 128x128 otherwise.  The 8-wave kernel from 100 tiles of
+    // 256x256, every format: there it measured faster than the 4-wave kernel on
+    // every block shape (int8 4096^2 109 vs 134 us, FF up 428 vs 472, FF down
+    // 405 vs 435; bf16 4096^2 91 vs 105, FF up 350 vs 420, FF down 339 vs 404,
+    // 1024 x 4096 -> 12320 87 vs 101).  (Two forms that are faster alone on the
+    // A2V query projection, 3456 x 4096 -> 2080, 126 tiles, stay explicit, as the
+    // step follows the CU time of its launches: 256x128 tiles, 14 % faster, the
+    // step 0.25 ms slower; 128-row tiles, 79 -> 61 us with 48 % more CU time, the
+    // step 1.0-1.6 ms slower.  The block asks for the 256-row tiles there.)
     const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256);
     const bool g8 = g8_ok<BKIND>(p);
     tile = big >= 160 ? (g8 ? 5 : 1) : (big >= 100 && g8 ? 5 : 2);
-    // row sums of squares come from the 8-wave kernels' epilogues only
+    // row sums of squares come from the mid-size and 8-wave kernels' epilogues
     if (p.rowss && tile != 5) tile = 5;
   }
   if (p.rowss && tile != 5 && tile != 6) return LTX_ERR_UNSUPPORTED;
@@ -1870,8 +1870,8 @@ extern "C" int ltx_gemm_mxfp8_bf16(const void* A, int64_t lda, const uint8_t* Wq
 // bf16 as ltx_gemm_bf16, 1: int8 as ltx_gemm_w8a16_bf16, 2: MXFP8 as
 // ltx_gemm_mxfp8_bf16) with the per-row sums of squares of its bf16 outputs in
 // columns [0, ss_cols): rowss[m * ld_rowss + j] = sum of C[m, n]^2 over
-// n in [64 j, 64 j + 64).  Always the 8-wave kernel (its epilogue computes
-// them); C is bit-identical to the plain entry point's on that kernel.
+// n in [64 j, 64 j + 64).  On the mid-size or the 8-wave kernel, whose epilogues
+// compute them; C is bit-identical to the plain entry point's on that kernel.
 extern "C" int ltx_gemm_rowss_bf16(int wformat, const void* A, int64_t lda, const void* W, int64_t ldw,
                                    const void* w_scale, int64_t ld_scale, const float* bias, void* C,
                                    int64_t ldc, int64_t M, int64_t N, int64_t K, int epilogue,

@@ -24,11 +24,14 @@
 // 384 x 4096 -> 16384 69.4 -> 59.3, 384 x 16384 -> 4096 105 -> 88, 1024 x
 // 16384 -> 4096 164 -> 144; 8-bit weights, whose activations were whole
 // lines already: 256 x 4096 -> 8192 MXFP8 27.1 -> 25.5, the rest within 3 %.)
-// What bounds it: a CU's operand bytes.  One CU streams at most 55-60 bytes
-// per ns of weights that come from HBM, however deep the ring (64-144 KB in
-// flight measured alike; 40 in 64-byte pieces), and ~110 of what the caches
-// hold, against a 128 x 128 tile's 384 (8-bit weights) or 512 (bf16) bytes
-// per k for 8 cycles of MFMA.
+// What bounds it: a CU's operand bytes, of which a 128 x 128 tile takes 384 (8-bit
+// weights) or 512 (bf16) per k for 8 cycles of MFMA.  With all CUs busy each gets
+// 47 bytes per ns, 12 TB/s together (384 x 4096 -> 16384 bf16 256 workgroups x
+// 2.6 MB in 56 us, 1296 x 4096 -> 4096 MXFP8 224 x 2.1 MB in 44), while the MFMAs
+// are busy 0.35-0.40 of the cycles, the LDS 0.17-0.19, and the L2 channels take
+// 0.3 requests per cycle; a few CUs alone get no more from HBM (bf16 26 x 188160
+// -> 2048, 16 workgroups: 43 bytes of weights per ns).  A deeper ring changed
+// nothing.
 #include "gemm_common.h"
 
 namespace ltx {
