@@ -113,15 +113,16 @@ def parse_args(argv=None):
                     help="stamp only the FF-up launches in the timed graphs (no per-class GEMM timing)")
     ap.add_argument("--cpu-runs", type=int, default=5, help="timed oracle block runs after one warmup")
     ap.add_argument("--counter-workload",
-                    choices=["ff-up", "ff-up-vs-library", "copy", "fused-ops", "attention", "audio-rows"],
+                    choices=["ff-up", "ff-up-vs-library", "copy", "fused-ops", "attention", "audio-rows", "mid-gemm"],
                     default=None,
                     help="run only a short workload for rocprofv3 --pmc passes and exit: the video FF "
                          "up-projection GEMM (4 launches, --weights format), the three row kernels (adaln, "
                          "gated add, QK-norm + RoPE; 4 cache-cold launches each), the video self-attention at "
                          "3456 and 6144 tokens and the 3456 x 256 text cross-attention (4 launches each, 32 "
                          "heads of 128, gated), the audio stream's four 68-row MXFP8 products (4 launches each "
-                         "on distinct weights, automatic split-K path then the one-launch few-row kernel) or a "
-                         "1 GiB device copy (3 launches, the FETCH_SIZE / WRITE_SIZE calibration)")
+                         "on distinct weights, automatic split-K path then the one-launch few-row kernel), "
+                         "two products of the mid-size kernel (384 x 4096 -> 16384 bf16, 1296 x 4096 -> 4096 "
+                         "MXFP8; 4 launches each on distinct weights) or a 1 GiB device copy (3 launches, the FETCH_SIZE / WRITE_SIZE calibration)")
     ap.add_argument("--counter-tile", choices=["auto", "256", "g8"], default="auto",
                     help="tile choice of the ff-up counter workload: the library's automatic choice (the "
                          "8-wave kernel for every format at this shape), the 4-wave 256x256 kernel, or the "
@@ -179,6 +180,14 @@ def counter_workload(kind: str, weights: str, tile_name: str = "auto") -> None:
                         gemm.linear_rows(x, wt, epilogue=epi, **kw)
                     else:
                         gemm.linear(x, wt, epilogue=epi, **kw)
+    elif kind == "mid-gemm":
+        g = torch.Generator(device="cuda").manual_seed(0)
+        for m, k, n, fmt in ((384, 4096, 16384, "bf16"), (1296, 4096, 4096, "mxfp8")):
+            x = torch.randn((m, k), generator=g, device="cuda").bfloat16()
+            wts = [gemm.make_weight((torch.randn((n, k), generator=g, device="cuda") * 0.02).bfloat16(),
+                                    torch.zeros(n, device="cuda"), kind=fmt) for _ in range(4)]
+            for wt in wts:
+                gemm.linear(x, wt)
     elif kind == "copy":
         src = torch.empty(1 << 30, dtype=torch.uint8, device="cuda")
         dst = torch.empty_like(src)
