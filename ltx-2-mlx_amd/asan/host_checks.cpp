@@ -245,6 +245,39 @@ int main(int argc, char** argv) {
   EXPECT(ltx_flash_attn_splitkv_noalloc_bf16(d, 4096, d, 4096, d, 32, d, 4096, nullptr, 0, 68, 3456, 32, 128,
                                              0.1f, 16, nullptr), LTX_ERR_INVALID_ARG);  // tk_pad below Tk
 
+  // timestep MLPs: descriptors are checked before any launch
+  ltx_adaln_mlp mlp{fd, d, fd, d, fd, d, fd, fo, fo, fo, 4096, 9, 1000.0f};
+  ltx_adaln_mlp mlps[9] = {mlp, mlp, mlp, mlp, mlp, mlp, mlp, mlp, mlp};
+  EXPECT(ltx_adaln_mlps_f32(nullptr, 1, nullptr), LTX_ERR_INVALID_ARG);
+  EXPECT(ltx_adaln_mlps_f32(mlps, -1, nullptr), LTX_ERR_INVALID_ARG);
+  EXPECT(ltx_adaln_mlps_f32(nullptr, 0, nullptr), LTX_OK);
+  EXPECT(ltx_adaln_mlps_f32(mlps, 9, nullptr), LTX_ERR_UNSUPPORTED);  // one call takes eight
+  for (int64_t dim : {int64_t(0), int64_t(12), int64_t(4104)}) {
+    mlps[1].dim = dim;
+    EXPECT(ltx_adaln_mlps_f32(mlps, 2, nullptr), dim == 0 ? LTX_ERR_INVALID_ARG : LTX_ERR_UNSUPPORTED);
+  }
+  mlps[1] = mlp;
+  mlps[1].num = int64_t(1) << 40;
+  EXPECT(ltx_adaln_mlps_f32(mlps, 2, nullptr), LTX_ERR_UNSUPPORTED);
+  mlps[1] = mlp;
+  mlps[1].w2 = m;
+  EXPECT(ltx_adaln_mlps_f32(mlps, 2, nullptr), LTX_ERR_ALIGNMENT);
+  mlps[1] = mlp;
+  mlps[1].h1 = nullptr;
+  EXPECT(ltx_adaln_mlps_f32(mlps, 2, nullptr), LTX_ERR_INVALID_ARG);
+
+  // automatic GEMM choices, also of sizes that no launch could take
+  for (int wf = -1; wf <= 3; ++wf) {
+    for (int64_t v : {int64_t(-1), int64_t(0), int64_t(1), int64_t(68), int64_t(188160), INT64_MAX / 4}) {
+      const int s = ltx_gemm_auto_splits(v, 2048, 188160, wf);
+      EXPECT(s >= 1 && s <= 64, 1);
+      EXPECT(ltx_gemm_auto_splits(68, v, v, wf) >= 1, 1);
+      const int r = ltx_gemm_auto_rows(v, 4096, 4096, wf, 1);
+      EXPECT(r == 0 || r == 64 || r == 128 || r == 192, 1);
+      EXPECT(ltx_gemm_auto_rows(68, 4096, 4096, wf, (int)(v & 0xff)) >= 0, 1);
+    }
+  }
+
   // ---- launch planning: valid calls, refused at the launch (no device).
   // Never with a device present: the fake addresses would reach a kernel.
   int ndev = 0;
@@ -272,12 +305,17 @@ int main(int argc, char** argv) {
         EXPECT(ltx_output_norm_modulate_bf16(d, c, fd, fd, d, c, rows, c, 1e-6f, nullptr), LTX_ERR_HIP);
       }
     }
+    // timestep MLPs: one, and a step's eight of both widths
+    mlps[1] = mlp;
+    for (int i = 0; i < 8; ++i) mlps[i].dim = i < 4 ? 4096 : 2048, mlps[i].num = i == 7 ? 1 : 9;
+    for (int64_t n : {int64_t(1), int64_t(8)}) EXPECT(ltx_adaln_mlps_f32(mlps, n, nullptr), LTX_ERR_HIP);
     // GEMMs: every tile choice on the block's shapes, the 68-row audio shapes
     // and the text-context shapes, every epilogue code
     struct Shape { int64_t m, n, k; };
     const Shape shapes[] = {{3456, 16384, 4096}, {3456, 4096, 16384}, {3456, 12320, 4096}, {3456, 2080, 4096},
                             {3456, 4096, 2048}, {68, 6176, 2048}, {68, 2048, 8192}, {256, 8192, 4096},
-                            {10368, 4096, 4096}, {1, 1024, 4096}};
+                            {10368, 4096, 4096}, {1, 1024, 4096}, {77, 2048, 188160}, {1296, 4096, 128},
+                            {68, 4096, 3840}, {1296, 4128, 4096}};
     for (const Shape& sh : shapes) {
       for (int tile = 0; tile <= 6; ++tile) {
         for (int epi = 0; epi <= 4; ++epi) {
@@ -290,7 +328,7 @@ int main(int argc, char** argv) {
                                      sh.n - 32, nullptr), LTX_ERR_HIP);
           EXPECT(ltx_gemm_mxfp8_bf16(d, sh.k, q8, sh.k, q8, sh.k / 32, fd, d, sh.n, sh.m, sh.n, sh.k,
                                      flags | LTX_GEMM_ROUND_THEN_BIAS, r, sh.n, g, sh.n - 32, nullptr),
-                 LTX_ERR_HIP);
+                 tile >= 5 && sh.k % 512 ? LTX_ERR_UNSUPPORTED : LTX_ERR_HIP);  // 8-wave: whole scale octets
         }
       }
       for (int splits : {1, 2, 4, 8, 16}) {
