@@ -188,8 +188,8 @@ class LTXModel:
 
         def table(d):
             if init == "empty":
-                return torch.zeros((2, d), device=dev)
-            return (torch.randn((2, d), generator=gen, device=dev) * 0.02).contiguous()
+                return torch.zeros((2, d), dtype=torch.float32, device=dev)
+            return (torch.randn((2, d), generator=gen, dtype=torch.float32, device=dev) * 0.02).contiguous()
 
         # preprocess / output heads (bf16 weights; small, kept unquantised)
         self.patchify_proj = linear_weight(vd, in_channels, **lin)
@@ -220,12 +220,12 @@ class LTXModel:
             self.transformer_blocks.append(BasicAVTransformerBlock(i, self.video_config, self.audio_config,
                                                                    norm_eps=norm_eps, weights=w))
         # per-step buffers
-        self._temb_v = torch.empty((ADA_ROWS, vd), device=dev)
-        self._emb_v = torch.empty(vd, device=dev)
+        self._temb_v = torch.empty((ADA_ROWS, vd), dtype=torch.float32, device=dev)
+        self._emb_v = torch.empty(vd, dtype=torch.float32, device=dev)
         self._ada_v = torch.empty_like(self.video_tables)
         if audio:
-            self._temb_a = torch.empty((ADA_ROWS, ad), device=dev)
-            self._emb_a = torch.empty(ad, device=dev)
+            self._temb_a = torch.empty((ADA_ROWS, ad), dtype=torch.float32, device=dev)
+            self._emb_a = torch.empty(ad, dtype=torch.float32, device=dev)
             self._ada_a = torch.empty_like(self.audio_tables)
         self._rope_cache: dict = {}
 
@@ -319,8 +319,8 @@ class LTXModel:
         g_n = len(groups.values)
         vals = torch.tensor(groups.values, dtype=torch.float32, device=dev)
         temb = self._temb_v.unsqueeze(0).repeat(g_n, 1, 1)
-        emb = torch.empty((g_n, d), device=dev)
-        ada = torch.empty((g_n,) + tuple(self._ada_v.shape), device=dev)
+        emb = torch.empty((g_n, d), dtype=torch.float32, device=dev)
+        ada = torch.empty((g_n,) + tuple(self._ada_v.shape), dtype=torch.float32, device=dev)
         stream = _lib.stream_of(ada)
         for g in range(g_n):
             flat = temb[g].view(-1)

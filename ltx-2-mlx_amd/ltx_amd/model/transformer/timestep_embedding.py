@@ -32,8 +32,8 @@ def run_mlps(jobs: list, scratch: list | None = None) -> None:
     for i in range(0, len(jobs), MAX_MLPS):
         part = jobs[i:i + MAX_MLPS]
         dev = part[0][3].device
-        rows = (torch.empty((len(part), 2, max(j[0].dim for j in part)), device=dev) if scratch is None
-                else scratch[i:i + MAX_MLPS])
+        rows = (torch.empty((len(part), 2, max(j[0].dim for j in part)), dtype=torch.float32, device=dev)
+                if scratch is None else scratch[i:i + MAX_MLPS])
         args = (_MlpArgs * len(part))()
         for a, h, (m, t, mult, out, embedded) in zip(args, rows, part):
             h2 = h[1] if embedded is None else embedded
@@ -54,11 +54,14 @@ class AdaLayerNormSingle:
                 return torch.empty(shape, dtype=torch.bfloat16, device=device)
             return (torch.randn(shape, generator=g, device=device, dtype=torch.float32) * std).to(torch.bfloat16)
 
+        def zeros(n):
+            return torch.zeros(n, dtype=torch.float32, device=device)
+
         self.dim = dim
         self.num_embeddings = num_embeddings
-        self.w1, self.b1 = rnd((dim, SINUSOID_DIM)), torch.zeros(dim, device=device)
-        self.w2, self.b2 = rnd((dim, dim)), torch.zeros(dim, device=device)
-        self.w, self.b = rnd((num_embeddings * dim, dim)), torch.zeros(num_embeddings * dim, device=device)
+        self.w1, self.b1 = rnd((dim, SINUSOID_DIM)), zeros(dim)
+        self.w2, self.b2 = rnd((dim, dim)), zeros(dim)
+        self.w, self.b = rnd((num_embeddings * dim, dim)), zeros(num_embeddings * dim)
 
     def nbytes(self) -> int:
         return sum(t.numel() * t.element_size() for t in (self.w1, self.b1, self.w2, self.b2, self.w, self.b))
