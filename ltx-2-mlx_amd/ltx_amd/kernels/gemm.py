@@ -419,8 +419,10 @@ def rowss_eligible(x: torch.Tensor, weight: LinearWeight) -> bool:
 def single_g8_round(x: torch.Tensor, weight: LinearWeight) -> bool:
     """Whether the product is one partial round of the 8-wave kernel (100-159
     tiles of 256x256), where the automatic choice may be the mid-size kernel."""
-    m = x.numel() // max(weight.in_features, 1)
-    return rowss_eligible(x, weight) and ((m + 255) // 256) * ((weight.out_features + 255) // 256) < 160
+    if not rowss_eligible(x, weight):
+        return False
+    m = x.numel() // weight.in_features
+    return ((m + 255) // 256) * ((weight.out_features + 255) // 256) < 160
 
 
 def linear_rowss(x: torch.Tensor, weight: LinearWeight, ss_cols: int, *, sigmoid_from: int | None = None,

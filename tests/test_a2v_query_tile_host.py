@@ -46,6 +46,12 @@ def test_query_tile(monkeypatch, kind):
         assert _projection(monkeypatch, tokens, kind, **q)[1] == gemm.TILE_AUTO
 
 
+def test_quantised_rows_have_no_choice():
+    weight = gemm.LinearWeight(kind="mxfp8", w=torch.empty((2080, 4096), dtype=torch.uint8))
+    rows = gemm.MxRows(torch.empty((3456, 4096), dtype=torch.uint8), torch.empty((3456, 128), dtype=torch.uint8))
+    assert not gemm.single_g8_round(rows, weight)
+
+
 def test_block_asks_for_it():
     """Every A2V core call of the block passes the tile."""
     import inspect
