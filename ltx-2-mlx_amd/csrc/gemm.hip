@@ -1551,7 +1551,9 @@ static int kg_rows(int bkind, int64_t M, int64_t N, int64_t K, int64_t splits, d
 // tiles models faster (2.1 us per 128 k measured; int8 2.4).  Measured, this
 // kernel against that one, K = 4096: 1728 x 4096 bf16 78 / 76, MXFP8 61 / 73;
 // 2048 x 4096 86 / 76, 67 / 77; 2304 x 4096 81 / 75, 81 / 75; 384 x 16384
-// 55 / 71, 51 / 76; 512 x 16384 93 / 77, 74 / 76; 700 x 12320 90 / 79, 86 / 77.
+// 55 / 71, 51 / 76; 512 x 16384 93 / 77, 74 / 76; 700 x 12320 90 / 79, 86 / 77;
+// 2816 x 2080 45 / 69, 46 / 72; 3456 x 2080 70 / 69, 62 / 72 (the A2V query
+// projection, for which the block asks for the 8-wave kernel: CU time).
 // Shallow products of more than one round of 64-row tiles keep the older
 // kernels: with one to three units the loop is over before the ring has filled,
 // and two 128x128 workgroups per CU hide one's first loads behind the other's
